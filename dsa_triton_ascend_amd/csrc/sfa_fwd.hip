@@ -62,10 +62,25 @@ struct SfaFwdParams {
   int32_t mode, layout_q, layout_kv;
   int64_t band_pre, band_next;  // pre_tokens / next_tokens clamped to +-kBandOpen
   int32_t max_blocks, page_size;
-  int32_t splits, rows_per_xcd, pos_per_split;
+  int32_t splits, pos_per_split;
+  int32_t row_shift;  // 2^row_shift consecutive rows go to one XCD in turn (sfa_block_row)
   float scale_log2;
   int32_t return_lse;  // 0: no statistics, 1: the statistics, 2: zeros
 };
+
+// Row of slot j of an XCD (workgroup x runs on XCD x % 8): blocks of
+// 2^row_shift consecutive rows go to the XCDs in turn, the last rows first.
+// Under a causal mask the first rows of a sequence are short: given one
+// contiguous range of rows each, XCD 0 ran out of work at a quarter of the
+// others' (4096 rows of up to 2048 tokens: 0.75 of the chip's time used,
+// 8192 rows: 0.875), and rows in ascending order left the longest ones for
+// the last round.  Blocks keep the rows that run together on an XCD adjacent
+// (neighbouring rows select much the same keys, which its L2 then holds).
+__device__ __forceinline__ int64_t sfa_block_row(const SfaFwdParams& p, int xcd, int j) {
+  const int sh = p.row_shift;
+  const int64_t i = (((int64_t)(j >> sh) * 8 + xcd) << sh) + (j & ((1 << sh) - 1));
+  return p.rows - 1 - i;
+}
 
 constexpr int kSfaTile = 32;
 constexpr int kSfaMaxList = 2048;
@@ -168,9 +183,9 @@ __global__ __launch_bounds__(NW * 64, 1) void sfa_fwd_kernel(SfaFwdParams p) {
   const int jj = bid >> 3;
   const int hg = jj % hgroups;
   const int jr = jj / hgroups;
-  const int64_t row = (int64_t)(bid & 7) * p.rows_per_xcd + jr / p.splits;
+  const int64_t row = sfa_block_row(p, bid & 7, jr / p.splits);
   const int split = jr % p.splits;
-  if (row >= p.rows) return;
+  if (row < 0) return;
 
   const RowInfo ri = sfa_row_info(p, (int)row);
   if (tid == 0) s_ri = ri;
@@ -288,7 +303,7 @@ __global__ __launch_bounds__(NW * 64, 1) void sfa_fwd_kernel(SfaFwdParams p) {
     int bl = blockIdx.x;
     asm volatile("" : "+s"(bl));
     const int jr2 = (bl >> 3) / hgroups;
-    const int64_t row2 = (int64_t)(bl & 7) * p.rows_per_xcd + jr2 / p.splits;
+    const int64_t row2 = sfa_block_row(p, bl & 7, jr2 / p.splits);
     const int q0 = (jr2 % p.splits) * p.pos_per_split;
     const int q1 = min(p.K * p.bs, q0 + p.pos_per_split);
     const RowInfo rc = s_ri;
@@ -857,9 +872,9 @@ __global__ __launch_bounds__(512, 1) void sfa_fwd_ds_kernel(SfaFwdParams p) {
   const int jj = bid >> 3;
   const int hg = jj % hgroups;
   const int jr = jj / hgroups;
-  const int64_t row = (int64_t)(bid & 7) * p.rows_per_xcd + jr / p.splits;
+  const int64_t row = sfa_block_row(p, bid & 7, jr / p.splits);
   const int split = jr % p.splits;
-  if (row >= p.rows) return;
+  if (row < 0) return;
 
   const RowInfo ri = sfa_row_info(p, (int)row);
   if (tid == 0) s_ri = ri;
@@ -976,7 +991,7 @@ __global__ __launch_bounds__(512, 1) void sfa_fwd_ds_kernel(SfaFwdParams p) {
     int bl = blockIdx.x;
     asm volatile("" : "+s"(bl));
     const int jr2 = (bl >> 3) / hgroups;
-    const int64_t row2 = (int64_t)(bl & 7) * p.rows_per_xcd + jr2 / p.splits;
+    const int64_t row2 = sfa_block_row(p, bl & 7, jr2 / p.splits);
     const int q0 = (jr2 % p.splits) * p.pos_per_split;
     const int q1 = min(p.K * p.bs, q0 + p.pos_per_split);
     const RowInfo rc = s_ri;
@@ -1444,14 +1459,13 @@ __global__ __launch_bounds__(256) void sfa_combine_kernel(SfaFwdParams p) {
   constexpr int PER = D / 64;
   typedef _Float16 hvec __attribute__((ext_vector_type(PER)));
   const int lane = threadIdx.x & 63;
-  // (row, head) of this wave, with the forward launch's XCD mapping (rows
-  // rows_per_xcd * x .. of XCD x = blockIdx & 7), so the partials a wave
-  // reads were written through the same XCD's L2
+  // (row, head) of this wave, with the forward launch's XCD mapping, so the
+  // partials a wave reads were written through the same XCD's L2
   const int bpr = (p.n1 + 3) / 4;  // blocks per row
   const int jb = (int)(blockIdx.x >> 3);
-  const int64_t crow = (int64_t)(blockIdx.x & 7) * p.rows_per_xcd + jb / bpr;
+  const int64_t crow = sfa_block_row(p, (int)(blockIdx.x & 7), jb / bpr);
   const int chead = (jb % bpr) * 4 + (int)(threadIdx.x >> 6);
-  if (crow >= p.rows || chead >= p.n1) return;
+  if (crow < 0 || chead >= p.n1) return;
   const int64_t rh = crow * p.n1 + chead;
   const int64_t sstride = p.rows * p.n1;  // (row, head) records per split
   if (p.splits <= 8) {
@@ -1677,11 +1691,24 @@ size_t sfa_fwd_workspace_bytes(int64_t rows, int64_t n1, int64_t d, int64_t tota
   return sfa_fwd_ws_for(sfa_fwd_splits_for(rows, n1, d, total_pos, one_list), rows, n1, d);
 }
 
+// Rows that go to one XCD in turn: 32 (one per CU of an XCD, so the rounds of
+// the CUs stay even), and below 256 rows the largest power of two that gives
+// every XCD the same number of rows.
+static int sfa_row_shift(int64_t rows) {
+  const int64_t rpx = (rows + 7) / 8;
+  int sh = 0;
+  while (sh < 5 && (rows >= 256 || rpx % (2ll << sh) == 0)) ++sh;
+  return sh;
+}
+static int64_t sfa_rows_per_xcd(const SfaFwdParams& p) {
+  const int64_t per_turn = 8ll << p.row_shift;
+  return ((p.rows + per_turn - 1) / per_turn) << p.row_shift;
+}
+
 template <int D, typename T>
 static hipError_t launch_sfa_fwd(SfaFwdParams& p, SfaFwdKind kind, hipStream_t stream) {
   const int heads_per_wg = kind == kFwdDs64 ? kSfaDsHeads : kSfaHeadsPerWg;
-  const int64_t rows_per_xcd = (p.rows + 7) / 8;
-  p.rows_per_xcd = (int)rows_per_xcd;
+  const int64_t rows_per_xcd = sfa_rows_per_xcd(p);
   const int64_t blocks = 8 * rows_per_xcd * p.splits * ((p.n1 + heads_per_wg - 1) / heads_per_wg);
   const bool buf = p.kv_rows * (int64_t)D * 2 < (1ll << 31) && !(test_flags() & kTestForceGlobalGather);
   using C = SfaCfg<D>;
@@ -1770,7 +1797,7 @@ int sfa_fwd_run(const void* query, const void* query_rope, const void* key, cons
   // 1: write the statistics; 2: write zeros to the caller's buffers (given
   // without return_lse), so that the caller needs no fill of its own
   p.return_lse = return_lse ? 1 : (softmax_max && softmax_sum ? 2 : 0);
-  p.rows_per_xcd = 0;
+  p.row_shift = sfa_row_shift(q_rows);
   hipError_t e;
   if (dtype == DSA_DTYPE_BF16) {
     e = d == 512 ? launch_sfa_fwd<512, bf16>(p, kind, stream)
