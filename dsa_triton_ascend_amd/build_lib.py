@@ -20,6 +20,7 @@ BUILD_DIR = os.path.join(ROOT, "_build")
 SOURCES = [
     "capi.cpp",
     "sfa_fwd.hip",
+    "sfa_fwd_few.hip",
     "sfa_bwd.hip",
     "li_fwd.hip",
     "kl_bwd.hip",

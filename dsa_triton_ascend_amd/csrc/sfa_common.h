@@ -95,8 +95,10 @@ __device__ __forceinline__ bool sfa_resolve_id(const P& p, const RowInfo& ri, in
   if (tok >= ri.hi || tok < ri.lo) return false;
   if (p.layout_kv == DSA_LAYOUT_PA_BSND) {
     if (tok >= (int64_t)p.max_blocks * p.page_size) return false;
-    int blk = tab[tok / p.page_size];
-    int64_t r = (int64_t)blk * p.page_size + tok % p.page_size;
+    // tok < ri.hi fits in 32 bits (a 64-bit division takes several times as long)
+    const unsigned pg = (unsigned)tok / (unsigned)p.page_size;
+    int blk = tab[pg];
+    int64_t r = (int64_t)blk * p.page_size + (int)((unsigned)tok - pg * (unsigned)p.page_size);
     *phys = (blk < 0 || r >= p.kv_rows) ? -1 : (int)r;
     return true;
   }

@@ -1,0 +1,91 @@
+// Parameters, row order and DMA helpers shared by the sparse flash attention
+// forward kernels (sfa_fwd.hip: 64 / 128 heads per workgroup; sfa_fwd_few.hip:
+// up to 32).
+#pragma once
+
+#include "common.h"
+#include "sfa_common.h"
+
+namespace dsa {
+
+struct SfaFwdParams {
+  const void* q;
+  const void* qr;
+  const void* k;
+  const void* kr;
+  const int32_t* idx;
+  const int32_t* act_q;
+  const int32_t* act_k;
+  const int32_t* block_table;
+  void* out;
+  float* smax;
+  float* ssum;
+  // split partials (splits > 1): part_o[s, r, h, :] = O_s / (l_s * scale_s)
+  // in fp16, scale_s = 2^e >= max |O_s / l_s| (so |values| < 1: fp16 keeps
+  // 11 bits for the largest ones); part_ml[s, r, h] = {reference max (log2
+  // units), l_s, exact max (log2 units), scale_s}
+  _Float16* part_o;
+  float* part_ml;
+  int64_t rows;
+  int64_t kv_rows;
+  int32_t batch, s1, s2, n1, K;
+  int32_t bs;  // sparse_block_size
+  int32_t mode, layout_q, layout_kv;
+  int64_t band_pre, band_next;  // pre_tokens / next_tokens clamped to +-kBandOpen
+  int32_t max_blocks, page_size;
+  int32_t splits, pos_per_split;
+  int32_t row_shift;  // 2^row_shift consecutive rows go to one XCD in turn (sfa_block_row)
+  float scale_log2;
+  int32_t return_lse;  // 0: no statistics, 1: the statistics, 2: zeros
+};
+
+// Row of slot j of an XCD (workgroup x runs on XCD x % 8): blocks of
+// 2^row_shift consecutive rows go to the XCDs in turn, the last rows first.
+// Under a causal mask the first rows of a sequence are short: given one
+// contiguous range of rows each, XCD 0 ran out of work at a quarter of the
+// others' (4096 rows of up to 2048 tokens: 0.75 of the chip's time used,
+// 8192 rows: 0.875), and rows in ascending order left the longest ones for
+// the last round.  Blocks keep the rows that run together on an XCD adjacent
+// (neighbouring rows select much the same keys, which its L2 then holds).
+__device__ __forceinline__ int64_t sfa_block_row(const SfaFwdParams& p, int xcd, int j) {
+  const int sh = p.row_shift;
+  const int64_t i = (((int64_t)(j >> sh) * 8 + xcd) << sh) + (j & ((1 << sh) - 1));
+  return p.rows - 1 - i;
+}
+
+// P carries a bf16 lo part (the P.V product then has ~16 bits of P) only
+// while a workgroup attends fewer tokens than this; from here on P is
+// rounded once to bf16, as the reference kernel rounds it
+// (sparse_flash_attention_triton.py:313-323).  The rounding error of O is
+// then ~2^-9 |v| / sqrt(3 n_eff) with n_eff the effective number of tokens
+// of the softmax, far below the fp32-golden tolerance (atol 2e-3) at these
+// lengths, while for a handful of tokens it is not.
+constexpr int kLoSplitMinTokens = 256;
+constexpr float kRefSlack = 64.f;  // log2 units
+// Smallest exponent of a split partial's scale 2^e: a partial whose largest
+// |O / l| is below 2^kPartMinExp (tiny values) keeps the scale 2^-120, so
+// the stored multiplier inv * 2^-e (inv <= 1: l counts the reference-max
+// token) stays finite and the stored values stay below 1.
+constexpr int kPartMinExp = -120;
+
+// One 16-byte-per-lane DMA from global memory straight into LDS: lane L's
+// 16 bytes land at lds_base + 16*L (LDS address taken from M0).  Issued via
+// inline asm so that the compiler does not drain all outstanding DMA before
+// every LDS read; the tile loop waits with explicit vmcnt counts instead.
+__device__ __forceinline__ void dma_buf16(unsigned lds_base, int voff, __amdgpu_buffer_rsrc_t rsrc) {
+  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, 0 offen lds"
+               :: "s"(lds_base), "v"(voff), "s"(rsrc) : "memory");
+}
+__device__ __forceinline__ void dma_glb16(unsigned lds_base, const void* gaddr) {
+  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off"
+               :: "s"(lds_base), "v"(gaddr) : "memory");
+}
+template <int N> __device__ __forceinline__ void wait_vmcnt() {
+  asm volatile("s_waitcnt vmcnt(%0)" :: "n"(N) : "memory");
+}
+
+// sfa_fwd_few.hip: D = 512 kernels for few heads (no token splits)
+int sfa_few_heads_per_wg(int64_t n1);
+hipError_t sfa_few_launch(const SfaFwdParams& p, int32_t dtype, bool buf, int64_t rows_per_xcd, hipStream_t stream);
+
+}  // namespace dsa

@@ -32,92 +32,15 @@
 #include <mutex>
 #include <type_traits>
 
-#include "common.h"
-#include "sfa_common.h"
+#include "sfa_fwd.h"
 
 namespace dsa {
 
-struct SfaFwdParams {
-  const void* q;
-  const void* qr;
-  const void* k;
-  const void* kr;
-  const int32_t* idx;
-  const int32_t* act_q;
-  const int32_t* act_k;
-  const int32_t* block_table;
-  void* out;
-  float* smax;
-  float* ssum;
-  // split partials (splits > 1): part_o[s, r, h, :] = O_s / (l_s * scale_s)
-  // in fp16, scale_s = 2^e >= max |O_s / l_s| (so |values| < 1: fp16 keeps
-  // 11 bits for the largest ones); part_ml[s, r, h] = {reference max (log2
-  // units), l_s, exact max (log2 units), scale_s}
-  _Float16* part_o;
-  float* part_ml;
-  int64_t rows;
-  int64_t kv_rows;
-  int32_t batch, s1, s2, n1, K;
-  int32_t bs;  // sparse_block_size
-  int32_t mode, layout_q, layout_kv;
-  int64_t band_pre, band_next;  // pre_tokens / next_tokens clamped to +-kBandOpen
-  int32_t max_blocks, page_size;
-  int32_t splits, pos_per_split;
-  int32_t row_shift;  // 2^row_shift consecutive rows go to one XCD in turn (sfa_block_row)
-  float scale_log2;
-  int32_t return_lse;  // 0: no statistics, 1: the statistics, 2: zeros
-};
-
-// Row of slot j of an XCD (workgroup x runs on XCD x % 8): blocks of
-// 2^row_shift consecutive rows go to the XCDs in turn, the last rows first.
-// Under a causal mask the first rows of a sequence are short: given one
-// contiguous range of rows each, XCD 0 ran out of work at a quarter of the
-// others' (4096 rows of up to 2048 tokens: 0.75 of the chip's time used,
-// 8192 rows: 0.875), and rows in ascending order left the longest ones for
-// the last round.  Blocks keep the rows that run together on an XCD adjacent
-// (neighbouring rows select much the same keys, which its L2 then holds).
-__device__ __forceinline__ int64_t sfa_block_row(const SfaFwdParams& p, int xcd, int j) {
-  const int sh = p.row_shift;
-  const int64_t i = (((int64_t)(j >> sh) * 8 + xcd) << sh) + (j & ((1 << sh) - 1));
-  return p.rows - 1 - i;
-}
-
 constexpr int kSfaTile = 32;
 constexpr int kSfaMaxList = 2048;
-// P carries a bf16 lo part (the P.V product then has ~16 bits of P) only
-// while a workgroup attends fewer tokens than this; from here on P is
-// rounded once to bf16, as the reference kernel rounds it
-// (sparse_flash_attention_triton.py:313-323).  The rounding error of O is
-// then ~2^-9 |v| / sqrt(3 n_eff) with n_eff the effective number of tokens
-// of the softmax, far below the fp32-golden tolerance (atol 2e-3) at these
-// lengths, while for a handful of tokens it is not.
-constexpr int kLoSplitMinTokens = 256;
-constexpr float kRefSlack = 64.f;  // log2 units
-// Smallest exponent of a split partial's scale 2^e: a partial whose largest
-// |O / l| is below 2^kPartMinExp (tiny values) keeps the scale 2^-120, so
-// the stored multiplier inv * 2^-e (inv <= 1: l counts the reference-max
-// token) stays finite and the stored values stay below 1.
-constexpr int kPartMinExp = -120;
-
 // Zero row for padding slots of the 64-bit gather path (the buffer path
 // gets zeros from the hardware range check instead).
 __device__ __attribute__((aligned(16))) unsigned char g_sfa_zero_row[1024];
-
-// One 16-byte-per-lane DMA from global memory straight into LDS: lane L's
-// 16 bytes land at lds_base + 16*L (LDS address taken from M0).  Issued via
-// inline asm so that the compiler does not drain all outstanding DMA before
-// every LDS read; the tile loop waits with explicit vmcnt counts instead.
-__device__ __forceinline__ void dma_buf16(unsigned lds_base, int voff, __amdgpu_buffer_rsrc_t rsrc) {
-  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, 0 offen lds"
-               :: "s"(lds_base), "v"(voff), "s"(rsrc) : "memory");
-}
-__device__ __forceinline__ void dma_glb16(unsigned lds_base, const void* gaddr) {
-  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off"
-               :: "s"(lds_base), "v"(gaddr) : "memory");
-}
-template <int N> __device__ __forceinline__ void wait_vmcnt() {
-  asm volatile("s_waitcnt vmcnt(%0)" :: "n"(N) : "memory");
-}
 
 // HT = head tiles (of 16 heads) per wave, NW = waves; a workgroup covers
 // NW*HT*16 heads.
@@ -1578,6 +1501,7 @@ template <int D> struct SfaCfg {
   static constexpr int HT = D >= 512 ? 1 : 2;
 };
 constexpr int kSfaHeadsPerWg = 128;
+constexpr int kSfaFewMaxHeads = 32;  // up to here D = 512 runs sfa_fwd_few.hip
 
 // Token splits: when the (row, head group) units fill fewer than half the
 // CUs, enough splits to fill them, with at least 256 positions per split.
@@ -1590,14 +1514,18 @@ constexpr int kSfaHeadsPerWg = 128;
 //
 // Kernel choice: D = 512 launches that split tokens with 64-head workgroups
 // run sfa_fwd_ds_kernel with 64 heads (decode: 44.8 us against 46.6 with
-// 128 heads and twice the splits); other D = 512 launches run it with 128
-// heads (each KV row gathered once per row; prefill 4.64 ms against 4.77
+// 128 heads and twice the splits), and so do up to 64 heads unsplit (8192
+// rows: 2.74 ms against 3.90 on 128-head workgroups); unsplit rows of up to 32
+// heads run sfa_fwd_few_kernel; other D = 512 launches run 128 heads per
+// workgroup (each KV row gathered once per row; prefill 4.64 ms against 4.77
 // for sfa_fwd_kernel); D < 512 runs sfa_fwd_kernel (128 heads).
 static int sfa_fwd_plan_splits(int64_t rows, int64_t n1, int64_t total_pos, int heads_per_wg) {
   const int cus = device_cu_count();
   const int64_t units = rows * ((n1 + heads_per_wg - 1) / heads_per_wg);
   if (2 * units > cus) return 1;
-  const int64_t want = (cus + units - 1) / units;
+  // one round of workgroups: 48 rows of 64 heads in 5 splits each 35 us; in 6,
+  // 288 workgroups took two rounds and 55 us
+  const int64_t want = cus / units;
   const int64_t by_len = (total_pos + 255) / 256;
   const int64_t splits = want < by_len ? want : by_len;
   return splits < 1 ? 1 : (int)splits;
@@ -1649,14 +1577,18 @@ int sfa_fwd_scratch(void** ptr) {
   return DSA_OK;
 }
 
-enum SfaFwdKind { kFwdWide, kFwdDs64, kFwdDs128 };
+enum SfaFwdKind { kFwdWide, kFwdDs64, kFwdDs128, kFwdFew };
 static SfaFwdKind sfa_fwd_kind(int64_t rows, int64_t n1, int64_t d, int64_t total_pos) {
   if (d != 512 || (test_flags() & kTestFwdWide)) return kFwdWide;
   if (sfa_fwd_plan_splits(rows, n1, total_pos, kSfaDsHeads) > 1) return kFwdDs64;
+  // few heads: enough rows, or enough tokens per row, for waves that work alone
+  if (n1 <= kSfaFewMaxHeads && (total_pos > 512 || rows > 2ll * device_cu_count())) return kFwdFew;
+  if (n1 <= kSfaDsHeads) return kFwdDs64;
   return kFwdDs128;
 }
 static int sfa_fwd_heads_per_wg(int64_t rows, int64_t n1, int64_t d, int64_t total_pos) {
-  return sfa_fwd_kind(rows, n1, d, total_pos) == kFwdDs64 ? kSfaDsHeads : kSfaHeadsPerWg;
+  const SfaFwdKind kind = sfa_fwd_kind(rows, n1, d, total_pos);
+  return kind == kFwdFew ? sfa_few_heads_per_wg(n1) : kind == kFwdDs64 ? kSfaDsHeads : kSfaHeadsPerWg;
 }
 
 static size_t sfa_fwd_ws_for(int64_t splits, int64_t rows, int64_t n1, int64_t d) {
@@ -1677,6 +1609,7 @@ constexpr size_t kSfaOneListMaxWs = 4ull << 30;
 static int sfa_fwd_splits_for(int64_t rows, int64_t n1, int64_t d, int64_t total_pos, bool one_list) {
   const int fill = sfa_fwd_plan_splits(rows, n1, total_pos, sfa_fwd_heads_per_wg(rows, n1, d, total_pos));
   if (!one_list || d != 512 || (test_flags() & kTestFwdWide)) return fill;
+  if (sfa_fwd_kind(rows, n1, d, total_pos) == kFwdFew) return fill;  // takes ranges of any length
   const int64_t need = (total_pos + kSfaMaxList - 1) / kSfaMaxList;
   if (need <= fill) return fill;
   if (sfa_fwd_ws_for(need, rows, n1, d) > kSfaOneListMaxWs) return fill;
@@ -1728,7 +1661,10 @@ static hipError_t launch_sfa_fwd(SfaFwdParams& p, SfaFwdKind kind, hipStream_t s
         hipLaunchKernelGGL((sfa_fwd_ds_kernel<D, T, HG, false, true>), grid, dim3(512), 0, stream, p);
     }
   };
-  if (kind == kFwdDs64) {
+  if (kind == kFwdFew) {
+    const hipError_t fe = sfa_few_launch(p, __is_same(T, bf16) ? DSA_DTYPE_BF16 : DSA_DTYPE_FP16, buf, rows_per_xcd, stream);
+    if (fe != hipSuccess) return fe;
+  } else if (kind == kFwdDs64) {
     launch_ds(std::integral_constant<int, 64>{});
   } else if (kind == kFwdDs128) {
     launch_ds(std::integral_constant<int, 128>{});
