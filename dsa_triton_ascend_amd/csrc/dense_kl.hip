@@ -18,11 +18,13 @@
 //
 // Design (the reference recomputes the index scores in all four kernels and
 // scatters dKi with fp32 atomics):
-//  * dense_index_kernel: one workgroup per query row streams the visible key
-//    index rows through LDS; 16 index heads per wave on MFMA, the weighted
-//    ReLU head-sum as an exact three-part bf16 product with a ones matrix.
-//    Writes I to a row-major fp32 buffer [rows, S2] and the row's LSE
-//    (online per thread, merged at the end).
+//  * dense_index_rows_kernel (D_idx = 128): four query rows per workgroup, one
+//    per wave, over shared 64-key tiles.  Writes I to a row-major fp32 buffer
+//    [rows, S2] and the row's LSE (online per lane, merged at the end).
+//  * dense_index_kernel (D_idx = 256, 512): one workgroup per query row streams
+//    the visible key index rows through LDS; 16 index heads per wave on MFMA,
+//    the weighted ReLU head-sum as an exact three-part bf16 product with a ones
+//    matrix.
 //  * dense_teacher_kernel: one workgroup per query row streams K / K_rope
 //    through a two-buffer LDS ring.  Waves 0-3 score 32 heads each on the
 //    32x32x16 MFMA (Q resident, one key row serves every head); waves 4-7
@@ -30,9 +32,12 @@
 //    - p against the index LSE, overwriting I in place; per-row loss.  For
 //    GQA the key heads are visited in turn and heads of other key heads
 //    are masked.
-//  * dense_index_grad_kernel: one workgroup per row: index scores again,
-//    dW in registers, dQi^T = Ki^T . dS^T through the transposing LDS read.
-//  * dense_dki_kernel: key-major.  A workgroup owns 128 keys (16 per wave,
+//  * dense_dqi_tile_kernel, dense_dki_tile_kernel (D_idx = 128, 32 / 64 / 128
+//    index heads): 32 resident columns per wave over shared 64-row tiles, below.
+//  * dense_index_grad_kernel (other shapes): one workgroup per row: index
+//    scores again, dW in registers, dQi^T = Ki^T . dS^T through the transposing
+//    LDS read.
+//  * dense_dki_kernel (other shapes): key-major.  A workgroup owns 128 keys (16 per wave,
 //    their index rows resident in registers as MFMA B operands) and a slice
 //    of the query rows that see them; per row it stages the row's index
 //    query in LDS 32 heads at a time, recomputes the ReLU mask, and
@@ -42,6 +47,8 @@
 // fp16 operands carry dS scaled by a per-row power of two (from the row's
 // max |dI| and max |w|) so that its hi / lo parts stay in the fp16 normal
 // range; products are scaled back in fp32.
+#include <algorithm>
+
 #include "kl_common.h"
 
 namespace dsa {
@@ -69,6 +76,7 @@ struct DkParams {
   void* dqi;
   void* dw;
   int32_t batch, s1, s2, n1, n2, g, nidx, w_dtype, splits;
+  int32_t chunk;       // query rows per dKi workgroup (tile kernels)
   float scale_log2;    // scale * log2(e)
 };
 
@@ -221,6 +229,139 @@ __global__ __launch_bounds__(kDkThreads, 1) void dense_index_kernel(DkParams p) 
     const float mm = wave_max(m);  // finite: the row has a visible key
     const float ss = wave_sum(m == -INFINITY ? 0.f : s * expf(m - mm));
     if (lane == 0 && p.imax_out) {
+      p.imax_out[row] = mm;
+      p.isum_out[row] = ss;
+    }
+  }
+}
+
+// ---------------------------------------------------------------------------
+// 64-key (or 64-head) tiles of 128-column rows by LDS-DMA, shared by the
+// kernels below: four waves, three buffers, tile t + 2 in flight during t
+// ---------------------------------------------------------------------------
+constexpr int kDkRowDi = 128;              // index head dim of the tile kernels
+constexpr int kDkTile64 = 64;
+constexpr int kDkTileBytes = kDkTile64 * kDkRowDi * 2;
+
+// Row r of a tile (256 bytes) holds its 16-byte chunk c at c ^ nope_swz(r).
+// Wave w of four issues rows 16 w .. 16 w + 15, four rows (1 KB) per DMA; rows
+// past the last one re-read it (their products are never used).
+__device__ __forceinline__ void dk_issue_tile(unsigned lds, const unsigned char* base, int row0, int last, int wave,
+                                              int lane) {
+#pragma unroll
+  for (int j = 0; j < 4; ++j) {
+    const int r = wave * 16 + j * 4 + (lane >> 4);
+    const unsigned char* src = base + (int64_t)min(row0 + r, last) * (kDkRowDi * 2) + ((lane & 15) ^ nope_swz(r)) * 16;
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off"
+                 :: "s"(lds + (wave * 4 + j) * 1024), "v"(src) : "memory");
+  }
+}
+constexpr int kDkTileDmas = 4;  // per wave
+// Waits for this wave's DMAs of a tile, whose successor's are in flight (any
+// later load or store only makes the wait longer), or for all of them.
+__device__ __forceinline__ void dk_wait_tile(bool next_in_flight) {
+  if (next_in_flight) asm volatile("s_waitcnt vmcnt(%0)" :: "n"(kDkTileDmas) : "memory");
+  else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+}
+
+// Index scores I and their LSE at D_idx = 128: one query row per wave, four
+// consecutive rows of a batch per workgroup sharing each 64-key tile.  A row's
+// NHT * 16 heads are resident MFMA A operands, so a key fragment read from LDS
+// feeds NHT products (one, in dense_index_kernel, whose eight waves split the
+// heads of one row: its LDS reads and three barriers per 32 keys took 459 us
+// at 4096 causal rows of 64 heads, this takes 125 us, 137 GFLOP: 1.1 PFLOP/s).  The
+// weighted ReLU head sum runs on the accumulators in fp32, the four 16-lane
+// groups' partial sums meet in two lane swaps, and lane l ends up with key l.
+template <int NHT, typename T>
+__global__ __launch_bounds__(256, NHT > 4 ? 2 : 3) void dense_index_rows_kernel(DkParams p) {
+  using E = Elem<T>;
+  using V8 = typename E::v8;
+  constexpr int KSI = kDkRowDi / 32, IROW = kDkRowDi * 2;
+  __shared__ __attribute__((aligned(1024))) unsigned char s_ki[3][kDkTileBytes];
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int li = lane & 15, lg = lane >> 4;
+  const int groups = (p.s1 + 3) / 4;
+  const int b = blockIdx.x % p.batch;
+  const int s0 = (groups - 1 - (int)(blockIdx.x / p.batch)) * 4;  // long causal rows first
+  const int aq = p.act_q ? p.act_q[b] : p.s1;
+  const int ak = p.act_k ? p.act_k[b] : p.s2;
+  auto vis_of = [&](int s1) { return s1 < aq && s1 < p.s1 ? min(max(ak - aq + s1 + 1, 0), p.s2) : 0; };
+  const int vis = vis_of(s0 + wave);
+  int top = 0;
+#pragma unroll
+  for (int w = 0; w < 4; ++w) top = max(top, vis_of(s0 + w));
+  const int nt = (top + kDkTile64 - 1) / kDkTile64;
+  const int row = b * p.s1 + s0 + wave;
+  const bool have = s0 + wave < p.s1;
+
+  const unsigned char* kib = (const unsigned char*)p.ki + (int64_t)b * p.s2 * IROW;
+  const unsigned ring = (unsigned)(uintptr_t)&s_ki[0][0];
+  if (nt > 0) dk_issue_tile(ring, kib, 0, p.s2 - 1, wave, lane);
+  if (nt > 1) dk_issue_tile(ring + kDkTileBytes, kib, kDkTile64, p.s2 - 1, wave, lane);
+  V8 qf[NHT][KSI];
+  float wr[NHT][4];
+  const u32x4 z4 = {0u, 0u, 0u, 0u};
+  const int64_t hrow = (int64_t)(have ? row : 0) * p.nidx;
+#pragma unroll
+  for (int ht = 0; ht < NHT; ++ht) {
+    const int g = ht * 16 + li;
+#pragma unroll
+    for (int ks = 0; ks < KSI; ++ks) {
+      const u32x4 v = *(const u32x4*)((const T*)p.qi + (hrow + min(g, p.nidx - 1)) * kDkRowDi + ks * 32 + lg * 8);
+      qf[ht][ks] = as_v8<V8>(g < p.nidx ? v : z4);
+    }
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      const int gg = ht * 16 + lg * 4 + r;
+      const float w = load_w(p.w, hrow + min(gg, p.nidx - 1), p.w_dtype);
+      wr[ht][r] = gg < p.nidx ? w : 0.f;
+    }
+  }
+  float m = -INFINITY, s = 0.f;  // online LSE of this lane's keys
+  int b3 = 0;
+  for (int t = 0; t < nt; ++t) {
+    dk_wait_tile(t + 1 < nt);
+    lds_barrier();
+    const int bn = b3 == 0 ? 2 : b3 - 1;  // the buffer of tile t - 1
+    if (t + 2 < nt) dk_issue_tile(ring + bn * kDkTileBytes, kib, (t + 2) * kDkTile64, p.s2 - 1, wave, lane);
+    if (t * kDkTile64 < vis) {
+      const unsigned char* buf = s_ki[b3];
+      float I = 0.f;
+#pragma unroll
+      for (int kt = 0; kt < 4; ++kt) {
+        f32x4 acc[NHT];
+#pragma unroll
+        for (int ht = 0; ht < NHT; ++ht) acc[ht] = (f32x4){0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int ks = 0; ks < KSI; ++ks) {
+          const int r = kt * 16 + li;
+          const V8 kf = as_v8<V8>(*(const u32x4*)(buf + r * IROW + (((ks * 4 + lg) ^ nope_swz(li)) * 16)));
+#pragma unroll
+          for (int ht = 0; ht < NHT; ++ht) acc[ht] = E::mfma(qf[ht][ks], kf, acc[ht]);
+        }
+        float a[4] = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int ht = 0; ht < NHT; ++ht)
+#pragma unroll
+          for (int r = 0; r < 4; ++r) a[r] = fmaf(relu_bits(acc[ht][r]), wr[ht][r], a[r]);
+        const float sum = xgroup_sum((a[0] + a[1]) + (a[2] + a[3]));
+        I = lg == kt ? sum : I;
+      }
+      const int key = t * kDkTile64 + lane;
+      if (key < vis) {
+        if (p.ibuf) p.ibuf[(int64_t)row * p.s2 + key] = I;
+        const float e = expf(-fabsf(I - m));
+        s = I > m ? fmaf(s, e, 1.f) : s + e;
+        m = I > m ? I : m;
+      }
+    }
+    b3 = b3 == 2 ? 0 : b3 + 1;
+  }
+  if (have && p.imax_out) {
+    const float mm = wave_max(m);  // -inf: the row has no visible key
+    const float ss = wave_sum(m == -INFINITY ? 0.f : s * expf(m - mm));
+    if (lane == 0) {
       p.imax_out[row] = mm;
       p.isum_out[row] = ss;
     }
@@ -754,6 +895,311 @@ __global__ __launch_bounds__(256) void dense_dki_reduce_kernel(const float* part
   *(T4*)(dki + 4 * i) = o;
 }
 
+// ---------------------------------------------------------------------------
+// D_idx = 128: dQi / dW and dKi on 64-row tiles, 32 resident columns per wave
+// ---------------------------------------------------------------------------
+// Both gradients are the same pair of products with rows and columns swapped:
+//   dots[tile row][column] = tile . resident^T, c = f(dots, dI, w),
+//   acc^T[d][column] += tile^T[d][tile row] . c[tile row][column]
+// (dQi: tile rows = keys, columns = a row's index heads; dKi: tile rows = a
+// row's index heads, columns = keys).  A wave holds 32 columns, so each
+// fragment read from LDS, plain or transposed, feeds two column tiles, and a
+// workgroup's four waves share the tile; with 16 columns per wave and one
+// 32-row tile between two barriers the two kernels took 547 and 769 us at 4096
+// causal rows of 64 heads (here 382 and 536; 412 GFLOP each, hi and lo parts
+// counted).  c goes to the second product as
+// hi + lo parts.  One half tile (32 rows) at a time: 48 MFMAs.
+constexpr int kDkCols = 32;
+
+template <typename T, bool SCALED, typename F>
+__device__ __forceinline__ void dk_half_tile(const unsigned char* half, const typename Elem<T>::v8 (&res)[2][4],
+                                             f32x4 (&acc)[kDkRowDi / 16][2], float unscale, int li, int lg, F&& value) {
+  using E = Elem<T>;
+  using V8 = typename E::v8;
+  constexpr int IROW = kDkRowDi * 2;
+  f32x4 dot[2][2];
+#pragma unroll
+  for (int c = 0; c < 2; ++c) dot[c][0] = dot[c][1] = (f32x4){0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+  for (int ks = 0; ks < 4; ++ks)
+#pragma unroll
+    for (int tt = 0; tt < 2; ++tt) {
+      const V8 a = as_v8<V8>(*(const u32x4*)(half + (tt * 16 + li) * IROW + (((ks * 4 + lg) ^ nope_swz(li)) * 16)));
+#pragma unroll
+      for (int c = 0; c < 2; ++c) dot[c][tt] = E::mfma(a, res[c][ks], dot[c][tt]);
+    }
+  // B operand of the second product: k = 8 lg + j is tile row 16 (j >> 2) + 4 lg + (j & 3)
+  V8 hi[2], lo[2];
+#pragma unroll
+  for (int c = 0; c < 2; ++c)
+#pragma unroll
+    for (int j = 0; j < 8; ++j) {
+      const float v = value(c, j >> 2, j & 3, dot[c][j >> 2][j & 3]);
+      const T h = E::from_f32(v);
+      hi[c][j] = h;
+      lo[c][j] = E::from_f32(v - E::to_f32(h));
+    }
+  const int r1 = lg * 4 + (li >> 2), hb = (li & 3) >> 1;
+#pragma unroll
+  for (int dt = 0; dt < kDkRowDi / 16; ++dt) {
+    const unsigned char* p1 = half + r1 * IROW + (((2 * dt + hb) ^ nope_swz(r1)) * 16) + (li & 1) * 8;
+    const i16x4 w1 = __builtin_bit_cast(i16x4, __builtin_amdgcn_ds_read_tr16_b64_v4bf16((lds_bf16x4*)p1));
+    const i16x4 w2 = __builtin_bit_cast(i16x4, __builtin_amdgcn_ds_read_tr16_b64_v4bf16((lds_bf16x4*)(p1 + 16 * IROW)));
+    const i16x8 w = {w1[0], w1[1], w1[2], w1[3], w2[0], w2[1], w2[2], w2[3]};
+    const V8 av = __builtin_bit_cast(V8, w);
+#pragma unroll
+    for (int c = 0; c < 2; ++c) {
+      if constexpr (SCALED) {
+        f32x4 t = E::mfma(av, hi[c], (f32x4){0.f, 0.f, 0.f, 0.f});
+        t = E::mfma(av, lo[c], t);
+        acc[dt][c] += t * unscale;
+      } else {
+        acc[dt][c] = E::mfma(av, hi[c], acc[dt][c]);
+        acc[dt][c] = E::mfma(av, lo[c], acc[dt][c]);
+      }
+    }
+  }
+}
+
+// dQi, dW: a workgroup's four waves take the 32-head groups of consecutive
+// rows (2 rows at 64 heads) over shared 64-key tiles.
+template <typename T>
+__global__ __launch_bounds__(256, 2) void dense_dqi_tile_kernel(DkParams p) {
+  using E = Elem<T>;
+  using V8 = typename E::v8;
+  constexpr int IROW = kDkRowDi * 2;
+  constexpr bool kF16 = __is_same(T, f16);
+  __shared__ __attribute__((aligned(1024))) unsigned char s_t[3][kDkTileBytes];
+  __shared__ __attribute__((aligned(16))) float s_di[4][kDkTile64];
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int li = lane & 15, lg = lane >> 4;
+  const int hgr = p.nidx / kDkCols, rpw = 4 / hgr;  // head groups per row, rows per workgroup
+  const int groups = (p.s1 + rpw - 1) / rpw;
+  const int b = blockIdx.x % p.batch;
+  const int s0 = (groups - 1 - (int)(blockIdx.x / p.batch)) * rpw;  // long causal rows first
+  const int s1 = s0 + wave / hgr, g0 = (wave % hgr) * kDkCols;
+  const int aq = p.act_q ? p.act_q[b] : p.s1;
+  const int ak = p.act_k ? p.act_k[b] : p.s2;
+  const bool have = s1 < p.s1;
+  const int row = b * p.s1 + (have ? s1 : 0);
+  auto vis_of = [&](int x) {
+    return x < aq && x < p.s1 && p.isum[b * p.s1 + x] > 0.f ? min(max(ak - aq + x + 1, 0), p.s2) : 0;
+  };
+  const int vis = vis_of(s1);
+  int top = 0;
+  for (int r = 0; r < rpw; ++r) top = max(top, vis_of(s0 + r));
+  const int nt = (top + kDkTile64 - 1) / kDkTile64;
+  const unsigned char* kib = (const unsigned char*)p.ki + (int64_t)b * p.s2 * IROW;
+  const unsigned ring = (unsigned)(uintptr_t)&s_t[0][0];
+  const float* irow = p.ibuf + (int64_t)row * p.s2;
+  float di_raw = irow[min(lane, p.s2 - 1)];  // masked where it is used
+  V8 res[2][4];
+  float wg[2], dw[2] = {0.f, 0.f};
+  const int64_t hrow = (int64_t)row * p.nidx + g0;
+  float scale = 1.f, unscale = 1.f;
+  if (kF16) {
+    const int e = p.dexp[row];
+    scale = ldexpf(1.f, e);
+    unscale = ldexpf(1.f, -e);
+  }
+#pragma unroll
+  for (int c = 0; c < 2; ++c) {
+#pragma unroll
+    for (int ks = 0; ks < 4; ++ks)
+      res[c][ks] = as_v8<V8>(*(const u32x4*)((const T*)p.qi + (hrow + c * 16 + li) * kDkRowDi + ks * 32 + lg * 8));
+    wg[c] = load_w(p.w, hrow + c * 16 + li, p.w_dtype);
+  }
+  if (nt > 0) dk_issue_tile(ring, kib, 0, p.s2 - 1, wave, lane);
+  if (nt > 1) dk_issue_tile(ring + kDkTileBytes, kib, kDkTile64, p.s2 - 1, wave, lane);
+  f32x4 acc[kDkRowDi / 16][2];
+#pragma unroll
+  for (int dt = 0; dt < kDkRowDi / 16; ++dt)
+#pragma unroll
+    for (int c = 0; c < 2; ++c) acc[dt][c] = (f32x4){0.f, 0.f, 0.f, 0.f};
+  int b3 = 0;
+  for (int t = 0; t < nt; ++t) {
+    s_di[wave][lane] = t * kDkTile64 + lane < vis ? di_raw : 0.f;
+    dk_wait_tile(t + 1 < nt);
+    lds_barrier();
+    di_raw = irow[min((t + 1) * kDkTile64 + lane, p.s2 - 1)];
+    const int bn = b3 == 0 ? 2 : b3 - 1;
+    if (t + 2 < nt) dk_issue_tile(ring + bn * kDkTileBytes, kib, (t + 2) * kDkTile64, p.s2 - 1, wave, lane);
+    if (t * kDkTile64 < vis) {
+#pragma unroll
+      for (int hh = 0; hh < 2; ++hh) {
+        f32x4 di[2];
+#pragma unroll
+        for (int tt = 0; tt < 2; ++tt) di[tt] = *(const f32x4*)&s_di[wave][hh * 32 + tt * 16 + lg * 4];
+        dk_half_tile<T, false>(s_t[b3] + hh * 32 * IROW, res, acc, 1.f, li, lg, [&](int c, int tt, int r, float dot) {
+          const float relu = relu_bits(dot);
+          dw[c] = fmaf(di[tt][r], relu, dw[c]);
+          return relu > 0.f ? di[tt][r] * wg[c] * scale : 0.f;
+        });
+      }
+    }
+    b3 = b3 == 2 ? 0 : b3 + 1;
+  }
+  if (!have) return;
+  typedef T T4 __attribute__((ext_vector_type(4)));
+#pragma unroll
+  for (int c = 0; c < 2; ++c) {
+    const float dwv = xgroup_sum(dw[c]);
+    if (lg == 0) store_w(p.dw, hrow + c * 16 + li, p.w_dtype, dwv);
+    T* dst = (T*)p.dqi + (hrow + c * 16 + li) * kDkRowDi;
+#pragma unroll
+    for (int dt = 0; dt < kDkRowDi / 16; ++dt) {
+      const T4 o = {E::from_f32(acc[dt][c][0] * unscale), E::from_f32(acc[dt][c][1] * unscale),
+                    E::from_f32(acc[dt][c][2] * unscale), E::from_f32(acc[dt][c][3] * unscale)};
+      *(T4*)(dst + dt * 16 + lg * 4) = o;
+    }
+  }
+}
+
+// dKi partials: a workgroup owns 128 keys (32 per wave) and p.chunk of the
+// query rows that see them.  The chunks have one length, so the workgroups'
+// work is even: with a fixed number of slices per key tile, the causal first
+// tiles' slices were 32 times as long as the last ones'.
+template <typename T>
+__global__ __launch_bounds__(256, 2) void dense_dki_tile_kernel(DkParams p) {
+  using E = Elem<T>;
+  using V8 = typename E::v8;
+  constexpr int IROW = kDkRowDi * 2;
+  constexpr bool kF16 = __is_same(T, f16);
+  __shared__ __attribute__((aligned(1024))) unsigned char s_t[3][kDkTileBytes];
+  __shared__ __attribute__((aligned(16))) float s_w[2][kDkTile64];
+  const int tid = threadIdx.x;
+  const int lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int li = lane & 15, lg = lane >> 4;
+  const int ntiles = (p.s2 + kDkKeys - 1) / kDkKeys;
+  // chunk `split` of key tile bt runs on XCD (bt - split) % 8: the first tiles
+  // have the most chunks, and each on an XCD of its own they gave XCD 0 half as
+  // much work again as XCD 7, a second round of workgroups
+  const int nt8 = (p.batch * ntiles + 7) / 8 * 8;
+  const int split = blockIdx.x / nt8, bt = (blockIdx.x - split * nt8 + split) % nt8;
+  if (bt >= p.batch * ntiles) return;
+  const int b = bt / ntiles, t0 = (bt - b * ntiles) * kDkKeys;
+  const int aq = p.act_q ? p.act_q[b] : p.s1;
+  const int ak = p.act_k ? p.act_k[b] : p.s2;
+  const int lo_all = max(0, t0 - ak + aq), hi_all = min(aq, p.s1);
+  const int r_lo = lo_all + split * p.chunk, r_hi = min(hi_all, r_lo + p.chunk);
+  if (r_lo >= r_hi) return;  // the reduction skips it too
+  // the chunk's index-query rows, 64 (row, head) pairs a tile
+  const int pairs = (r_hi - r_lo) * p.nidx;
+  const int nt = (pairs + kDkTile64 - 1) / kDkTile64;
+  const int64_t pair0 = ((int64_t)b * p.s1 + r_lo) * p.nidx;
+  const unsigned char* qib = (const unsigned char*)p.qi + pair0 * IROW;
+  const unsigned ring = (unsigned)(uintptr_t)&s_t[0][0];
+  V8 res[2][4];
+  int key[2];
+#pragma unroll
+  for (int c = 0; c < 2; ++c) {
+    key[c] = t0 + wave * kDkCols + c * 16 + li;
+    const int64_t kr = (int64_t)b * p.s2 + min(key[c], p.s2 - 1);
+#pragma unroll
+    for (int ks = 0; ks < 4; ++ks) res[c][ks] = as_v8<V8>(*(const u32x4*)((const T*)p.ki + kr * kDkRowDi + ks * 32 + lg * 8));
+  }
+  dk_issue_tile(ring, qib, 0, pairs - 1, wave, lane);
+  if (nt > 1) dk_issue_tile(ring + kDkTileBytes, qib, kDkTile64, pairs - 1, wave, lane);
+  // half tile h (32 pairs) belongs to one query row; dI of the lane's keys
+  // there, zero where the row does not see them (the teacher kernel wrote
+  // every visible key of the row).  Loaded a tile ahead, at addresses that
+  // wait for nothing: with a test of the row's index sum in front of them the
+  // loads cost each tile two memory round trips.
+  const int hsh = p.nidx == 32 ? 0 : p.nidx == 64 ? 1 : 2;
+  auto row_of = [&](int h) { return min(r_lo + (h >> hsh), r_hi - 1); };
+  float di[2][2];
+  // unconditional loads of raw values, masked and converted where they are
+  // used: a select right behind a load waits for it on the spot
+  auto load_di = [&](int t, float (&d)[2][2]) {
+#pragma unroll
+    for (int hh = 0; hh < 2; ++hh) {
+      const float* irow = p.ibuf + ((int64_t)b * p.s1 + row_of(2 * t + hh)) * p.s2;
+#pragma unroll
+      for (int c = 0; c < 2; ++c) d[hh][c] = irow[min(key[c], p.s2 - 1)];
+    }
+  };
+  const bool w32 = p.w_dtype == DSA_DTYPE_FP32;
+  const unsigned char* wb = (const unsigned char*)p.w + pair0 * (w32 ? 4 : 2);
+  auto load_wt = [&](int t) -> unsigned {  // the 32-bit word with weight 64 t + lane
+    const int i = min(t * kDkTile64 + lane, pairs - 1);
+    return *(const unsigned*)(wb + (w32 ? i * 4 : (i & ~1) * 2));
+  };
+  auto weight = [&](unsigned v) -> float {
+    if (w32) return __uint_as_float(v);
+    const unsigned short h = (unsigned short)(lane & 1 ? v >> 16 : v);  // tiles start at even weights
+    return p.w_dtype == DSA_DTYPE_BF16 ? __uint_as_float((unsigned)h << 16) : (float)__builtin_bit_cast(f16, h);
+  };
+  load_di(0, di);
+  unsigned wraw = load_wt(0);
+  f32x4 acc[kDkRowDi / 16][2];
+#pragma unroll
+  for (int dt = 0; dt < kDkRowDi / 16; ++dt)
+#pragma unroll
+    for (int c = 0; c < 2; ++c) acc[dt][c] = (f32x4){0.f, 0.f, 0.f, 0.f};
+  int b3 = 0;
+  for (int t = 0; t < nt; ++t) {
+    if (wave == 0) s_w[t & 1][lane] = weight(wraw);
+    dk_wait_tile(t + 1 < nt);
+    lds_barrier();
+    float dn[2][2];
+    wraw = load_wt(min(t + 1, nt - 1));
+    load_di(min(t + 1, nt - 1), dn);
+    const int bn = b3 == 0 ? 2 : b3 - 1;
+    if (t + 2 < nt) dk_issue_tile(ring + bn * kDkTileBytes, qib, (t + 2) * kDkTile64, pairs - 1, wave, lane);
+#pragma unroll
+    for (int hh = 0; hh < 2; ++hh) {
+      if ((2 * t + hh) * kDkCols >= pairs) break;
+      const int vis = min(max(ak - aq + row_of(2 * t + hh) + 1, 0), p.s2);
+      const float dv[2] = {key[0] < vis ? di[hh][0] : 0.f, key[1] < vis ? di[hh][1] : 0.f};
+      float scale = 1.f, unscale = 1.f;
+      if (kF16) {
+        const int e = p.dexp[b * p.s1 + row_of(2 * t + hh)];
+        scale = ldexpf(1.f, e);
+        unscale = ldexpf(1.f, -e);
+      }
+      f32x4 w[2];
+#pragma unroll
+      for (int tt = 0; tt < 2; ++tt) w[tt] = *(const f32x4*)&s_w[t & 1][hh * 32 + tt * 16 + lg * 4];
+      dk_half_tile<T, kF16>(s_t[b3] + hh * 32 * IROW, res, acc, unscale, li, lg, [&](int c, int tt, int r, float dot) {
+        return dot > 0.f ? dv[c] * w[tt][r] * scale : 0.f;
+      });
+    }
+#pragma unroll
+    for (int hh = 0; hh < 2; ++hh)
+#pragma unroll
+      for (int c = 0; c < 2; ++c) di[hh][c] = dn[hh][c];
+    b3 = b3 == 2 ? 0 : b3 + 1;
+  }
+#pragma unroll
+  for (int c = 0; c < 2; ++c) {
+    if (key[c] >= p.s2) continue;
+    float* dst = p.part + ((int64_t)split * p.batch * p.s2 + (int64_t)b * p.s2 + key[c]) * kDkRowDi;
+#pragma unroll
+    for (int dt = 0; dt < kDkRowDi / 16; ++dt) *(f32x4*)(dst + dt * 16 + lg * 4) = acc[dt][c];
+  }
+}
+
+// the chunks of a key's tile, in order
+template <typename T>
+__global__ __launch_bounds__(256) void dense_dki_tile_reduce_kernel(DkParams p, T* dki) {
+  const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
+  const int64_t n4 = (int64_t)p.batch * p.s2 * kDkRowDi / 4;
+  if (i >= n4) return;
+  const int64_t kr = i / (kDkRowDi / 4);
+  const int b = (int)(kr / p.s2), t0 = (int)(kr - (int64_t)b * p.s2) / kDkKeys * kDkKeys;
+  const int aq = p.act_q ? p.act_q[b] : p.s1;
+  const int ak = p.act_k ? p.act_k[b] : p.s2;
+  const int cnt = min(aq, p.s1) - max(0, t0 - ak + aq);
+  const int splits = cnt > 0 ? (cnt + p.chunk - 1) / p.chunk : 0;
+  f32x4 s = {0.f, 0.f, 0.f, 0.f};
+  for (int j = 0; j < splits; ++j) s += __builtin_nontemporal_load((const f32x4*)(p.part + ((int64_t)j * n4 + i) * 4));
+  typedef T T4 __attribute__((ext_vector_type(4)));
+  const T4 o = {Elem<T>::from_f32(s[0]), Elem<T>::from_f32(s[1]), Elem<T>::from_f32(s[2]), Elem<T>::from_f32(s[3])};
+  *(T4*)(dki + 4 * i) = o;
+}
+
 // loss = sum of the per-row terms in a fixed order (one workgroup)
 __global__ __launch_bounds__(256) void dense_loss_kernel(const float* part, int rows, float* loss) {
   __shared__ double s[256];
@@ -783,6 +1229,28 @@ int dense_kl_splits(int64_t batch, int64_t s1, int64_t s2) {
   return (int)sp;
 }
 
+// The tile kernels take D_idx = 128 and whole 32-head groups that divide four.
+static bool dk_tiles(int64_t nidx, int64_t di) { return di == kDkRowDi && (nidx == 32 || nidx == 64 || nidx == 128); }
+
+// Query rows per dKi workgroup, at least 32: one round of two workgroups per
+// CU over the (key tile, visible rows) of full-length sequences, counting a
+// shorter last chunk for each key tile (528 chunks on 512 slots would take
+// two rounds).
+static int dk_chunk(int64_t batch, int64_t s1, int64_t s2) {
+  // key tile i has min(s1, s2 - kDkKeys i) rows: all s1 in the first `full` tiles
+  const int64_t n = (s2 + kDkKeys - 1) / kDkKeys;
+  const int64_t full = s2 >= s1 ? std::min(n, (s2 - s1) / kDkKeys + 1) : 0;
+  const int64_t total = full * s1 + (n - full) * s2 - kDkKeys * ((n * (n - 1) - full * (full - 1)) / 2);
+  const int64_t cus = device_cu_count(), wgs = std::max(cus, 2 * cus - batch * n);
+  return (int)std::min<int64_t>(1 << 20, std::max<int64_t>(32, (batch * total + wgs - 1) / wgs));
+}
+static int64_t dk_part_splits(int64_t batch, int64_t s1, int64_t s2, int64_t di) {
+  const int64_t sp = dense_kl_splits(batch, s1, s2);
+  if (di != kDkRowDi) return sp;
+  const int64_t chunk = dk_chunk(batch, s1, s2);
+  return std::max<int64_t>(sp, (s1 + chunk - 1) / chunk);
+}
+
 struct DkWs {
   size_t ibuf, imax, isum, loss, dexp, part, total;
 };
@@ -802,7 +1270,7 @@ static DkWs dk_ws_layout(int64_t batch, int64_t s1, int64_t s2, int64_t di) {
   L.dexp = o;
   o += dk_align((size_t)rows * sizeof(int32_t));
   L.part = o;
-  o += dk_align((size_t)dense_kl_splits(batch, s1, s2) * batch * s2 * di * sizeof(float));
+  o += dk_align((size_t)dk_part_splits(batch, s1, s2, di) * batch * s2 * di * sizeof(float));
   L.total = o;
   return L;
 }
@@ -814,8 +1282,12 @@ size_t dense_kl_workspace_bytes(int64_t batch, int64_t s1, int64_t s2, int64_t d
 template <typename T>
 static hipError_t dk_index(const DkParams& p, int di, hipStream_t stream) {
   const dim3 grid((unsigned)(p.batch * p.s1));
-  if (di == 128) hipLaunchKernelGGL((dense_index_kernel<128, T>), grid, dim3(kDkThreads), 0, stream, p);
-  else if (di == 256) hipLaunchKernelGGL((dense_index_kernel<256, T>), grid, dim3(kDkThreads), 0, stream, p);
+  if (di == kDkRowDi) {
+    const dim3 g4((unsigned)(p.batch * ((p.s1 + 3) / 4)));
+    if (p.nidx <= 32) hipLaunchKernelGGL((dense_index_rows_kernel<2, T>), g4, dim3(256), 0, stream, p);
+    else if (p.nidx <= 64) hipLaunchKernelGGL((dense_index_rows_kernel<4, T>), g4, dim3(256), 0, stream, p);
+    else hipLaunchKernelGGL((dense_index_rows_kernel<8, T>), g4, dim3(256), 0, stream, p);
+  } else if (di == 256) hipLaunchKernelGGL((dense_index_kernel<256, T>), grid, dim3(kDkThreads), 0, stream, p);
   else hipLaunchKernelGGL((dense_index_kernel<512, T>), grid, dim3(kDkThreads), 0, stream, p);
   return hipGetLastError();
 }
@@ -840,6 +1312,17 @@ static hipError_t dk_grads(const DkParams& p, int di, void* d_key_index, hipStre
   const dim3 rgrid((unsigned)(p.batch * p.s1)), blk(kDkThreads);
   const int64_t ntiles = (p.s2 + kDkKeys - 1) / kDkKeys;
   const dim3 kgrid((unsigned)(p.batch * ntiles * p.splits));
+  if (dk_tiles(p.nidx, di)) {
+    const int rpw = 4 / (p.nidx / kDkCols);
+    hipLaunchKernelGGL((dense_dqi_tile_kernel<T>), dim3((unsigned)(p.batch * ((p.s1 + rpw - 1) / rpw))), dim3(256), 0,
+                       stream, p);
+    const int64_t chunks = (p.s1 + p.chunk - 1) / p.chunk;
+    hipLaunchKernelGGL((dense_dki_tile_kernel<T>), dim3((unsigned)((p.batch * ntiles + 7) / 8 * 8 * chunks)), dim3(256), 0, stream, p);
+    const int64_t n4t = (int64_t)p.batch * p.s2 * di / 4;
+    hipLaunchKernelGGL((dense_dki_tile_reduce_kernel<T>), dim3((unsigned)((n4t + 255) / 256)), dim3(256), 0, stream, p,
+                       (T*)d_key_index);
+    return hipGetLastError();
+  }
   if (di == 128) {
     hipLaunchKernelGGL((dense_index_grad_kernel<128, T>), rgrid, blk, 0, stream, p);
     hipLaunchKernelGGL((dense_dki_kernel<128, T>), kgrid, blk, 0, stream, p);
@@ -911,6 +1394,7 @@ int dense_kl_run(const void* query, const void* key, const void* query_rope, con
   p.dexp = (int32_t*)(ws + L.dexp);
   p.part = (float*)(ws + L.part);
   p.splits = dense_kl_splits(batch, s1, s2);
+  p.chunk = dk_chunk(batch, s1, s2);
   p.dqi = d_query_index;
   p.dw = d_weights;
   // the index scores always; their LSE unless the caller gives it

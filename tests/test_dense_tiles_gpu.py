@@ -1,0 +1,59 @@
+"""The D_idx = 128 kernels of the dense stage at the edges of their 64-row
+tiles, 128-key workgroups and query-row chunks: lengths around the tile sizes,
+several rows per workgroup, more keys than queries and the reverse, batches
+with hidden rows, 16-bit weights at an odd element offset.  Oracle, tolerances
+and their reasons: test_dense_kl_gpu."""
+import numpy as np
+import pytest
+import torch
+
+from oracle.dense_kl import dense_kl_bwd
+from tests.test_dense_kl_gpu import _case, _check, _dev, _np, _run
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16], ids=["bf16", "fp16"])
+@pytest.mark.parametrize("Ni", [32, 64, 128])
+@pytest.mark.parametrize("S1,S2", [(1, 1), (5, 63), (64, 64), (65, 129), (130, 193), (200, 70)])
+def test_tile_edges(S1, S2, Ni, dtype):
+    print(f"[dense tiles] S1={S1} S2={S2} Ni={Ni} {dtype}", flush=True)
+    c = _case(1, S1, S2, 32, 1, 128, Ni, 128, dtype, torch.float32)
+    got = _run(c, dtype, torch.float32, given_lse=False)
+    q, k, qr, kr, qi, ki, w, smax, ssum, scale = c
+    exp = dense_kl_bwd(q, k, qr, kr, qi, ki, w, smax, ssum, scale)
+    _check(got, exp, f"{S1}x{S2} Ni={Ni}", torch.float32)
+
+
+@pytest.mark.parametrize("Ni", [32, 128])
+def test_lengths_over_batches(Ni):
+    B, S1, S2 = 3, 70, 150
+    aq, ak = [70, 33, 1], [150, 20, 131]
+    print(f"[dense tiles] lengths Ni={Ni}", flush=True)
+    c = _case(B, S1, S2, 32, 1, 128, Ni, 128, torch.bfloat16, torch.bfloat16, aq, ak)
+    got = _run(c, torch.bfloat16, torch.bfloat16, given_lse=True, act_q=aq, act_k=ak)
+    q, k, qr, kr, qi, ki, w, smax, ssum, scale = c
+    exp = dense_kl_bwd(q, k, qr, kr, qi, ki, w, smax, ssum, scale, act_q=aq, act_k=ak)
+    _check(got, exp, f"lengths Ni={Ni}", torch.bfloat16)
+    for b in range(B):
+        assert np.all(got[0][b, aq[b]:] == 0) and np.all(got[2][b, aq[b]:] == 0) and np.all(got[1][b, ak[b]:] == 0)
+
+
+@pytest.mark.parametrize("w_dtype", [torch.bfloat16, torch.float16])
+def test_weights_at_an_odd_offset(w_dtype):
+    """16-bit weights that start two bytes past a word boundary."""
+    import dsa_triton_ascend_amd as dsa
+    print(f"[dense tiles] odd offset {w_dtype}", flush=True)
+    c = _case(1, 66, 140, 32, 1, 128, 64, 128, w_dtype, w_dtype)
+    q, k, qr, kr, qi, ki, w, smax, ssum, scale = c
+    d = [_dev(x, w_dtype) for x in (q, k, qi, ki)]
+    buf = torch.empty(w.size + 1, dtype=w_dtype, device="cuda")
+    odd = buf[1:].view(w.shape)
+    odd.copy_(_dev(w, w_dtype))
+    assert odd.is_contiguous() and odd.data_ptr() % 4 == 2
+    kw = dict(scale_value=scale, query_rope=_dev(qr, w_dtype), key_rope=_dev(kr, w_dtype))
+    st = (_dev(smax, torch.float32), _dev(ssum, torch.float32))
+    a = dsa.dense_loss_backward_triton(d[0], d[1], d[2], d[3], odd, *st, **kw)
+    b = dsa.dense_loss_backward_triton(d[0], d[1], d[2], d[3], _dev(w, w_dtype), *st, **kw)
+    for x, y in zip(a, b):
+        assert np.array_equal(_np(x), _np(y))
