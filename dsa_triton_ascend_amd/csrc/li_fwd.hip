@@ -1232,13 +1232,12 @@ __device__ void topk_row_generic(const TopkParams& p, const int64_t row, unsigne
 
 // ---------------------------------------------------------------------------
 // Fast selection, one workgroup per row of up to kFastMaxS2 scores, each
-// thread holding its kFastKpt keys in registers:
-//  1. n_valid, kmin and kmax of the row's finite keys.  All of them share the
-//     key bits above hb = bit length of (kmin ^ kmax).
-//  2. A 4096-bin histogram of the 12 key bits right below that common prefix;
-//     a scan from the top bin gives every bin's start in descending order
-//     and the bin b* that holds the take-th largest key.  The answer lies
-//     among the keys of bins >= b* (the candidates).
+// thread holding its KPT keys in registers:
+//  1. n_valid and kmax of the row's finite keys, and a floor under the answer.
+//  2. A histogram of the keys from the floor up, 4096 bins of 2^shift keys over
+//     [floor, kmax]; a scan from the top bin gives every bin's start in
+//     descending order and the bin b* that holds the take-th largest key.  The
+//     answer lies among the keys of bins >= b* (the candidates).
 //  3. Counting sort of the candidates by bin: each takes a slot in its bin's
 //     range (one LDS atomic per candidate).
 //  4. Within its bin, a candidate's final position is its rank by
@@ -1248,15 +1247,14 @@ __device__ void topk_row_generic(const TopkParams& p, const int64_t row, unsigne
 // more than kSegCap keys (crowded keys, e.g. many equal scores), take the
 // general path above.
 // ---------------------------------------------------------------------------
-constexpr int kFastKpt = 32;                            // keys per thread
-constexpr int kFastMaxS2 = kFastKpt * kTopkThreads;     // 32768
+constexpr int kFastMaxS2 = 32 * kTopkThreads;           // the widest variant: 32 keys per thread
 constexpr int kFastCap = 4096;                          // candidates (>= the largest K)
 constexpr int kFastBins = 4096;                         // 12-bit digits
 constexpr int kSegCap = 256;                            // keys per bin ranked directly
 constexpr int kTopkWaves = kTopkThreads / 64;
 // LDS of the fast path: bin counts, bin starts, bin cursors, candidate and
 // output buffers, misc words
-constexpr size_t kFastLds = 3 * (size_t)kFastBins * 4 + 2 * (size_t)kFastCap * 8 + 64 * 4;
+constexpr size_t kFastLds = 3 * (size_t)kFastBins * 4 + 2 * (size_t)kFastCap * 8 + 68 * 4;
 
 // Wave-wide operations on DPP lane moves (no LDS round trips).  DPP controls
 // of GFX9: row_shr:n = 0x110 + n, row_bcast:15 = 0x142, row_bcast:31 =
@@ -1308,7 +1306,10 @@ __device__ __forceinline__ void block_scan4(unsigned (&v)[4], unsigned* wsum) {
   }
 }
 
-template <bool IN_LDS>
+// KPT: keys per thread, 1024 * KPT >= the row (in 32-key threads a 9 K row spent
+// three quarters of its loads and compares on padding: the indexer step of 16
+// rows over 9001 keys 24.9 -> 22.7 us, of 32 rows over 3000 keys 24.7 -> 21.3).
+template <bool IN_LDS, int KPT>
 __global__ __launch_bounds__(kTopkThreads) void li_topk_kernel(TopkParams p) {
   extern __shared__ __attribute__((aligned(16))) unsigned char tk_smem[];
   const int64_t row = blockIdx.x;
@@ -1327,16 +1328,17 @@ __global__ __launch_bounds__(kTopkThreads) void li_topk_kernel(TopkParams p) {
   unsigned long long* const outb = cand + kFastCap;    // kFastCap
   unsigned* const misc = (unsigned*)(outb + kFastCap); // 48 words
   unsigned* const wsum = misc + 48;                    // kTopkWaves
+  unsigned* const s_big = wsum + kTopkWaves;           // the largest candidate bin
 
   // the row in registers, all loads in flight: 16-byte loads where the row
   // is 16-byte aligned (key u = 4q + e is entry 4 * (q * 1024 + tid) + e),
   // else entry u * 1024 + tid
   const bool vec = (((uintptr_t)srow & 15) == 0);
   auto entry = [&](int u) { return vec ? 4 * ((u >> 2) * kTopkThreads + tid) + (u & 3) : u * kTopkThreads + tid; };
-  unsigned kr[kFastKpt];
+  unsigned kr[KPT];
   if (vec) {
 #pragma unroll
-    for (int q = 0; q < kFastKpt / 4; ++q) {
+    for (int q = 0; q < KPT / 4; ++q) {
       const int j = 4 * (q * kTopkThreads + tid);
       float4 v = make_float4(-INFINITY, -INFINITY, -INFINITY, -INFINITY);
       if (j + 3 < S) {
@@ -1353,86 +1355,96 @@ __global__ __launch_bounds__(kTopkThreads) void li_topk_kernel(TopkParams p) {
     }
   } else {
 #pragma unroll
-    for (int u = 0; u < kFastKpt; ++u) {
+    for (int u = 0; u < KPT; ++u) {
       const int j = u * kTopkThreads + tid;
       kr[u] = j < S ? sort_key(srow[j]) : kNegInfKey;
     }
   }
   for (int i = tid; i < kFastBins; i += kTopkThreads) hcount[i] = 0u;
 
-  // ---- 1. count and range of the finite keys ----
+  // ---- 1. count and range of the finite keys, and a floor under the answer ----
+  // The smallest of the threads' t-th largest keys, t = K / threads rounded
+  // up, has at least K keys at or above it: keys below it are never selected.
+  // With 32 keys per thread and t = 2 it leaves about a quarter of the keys to
+  // count (their LDS atomics were the histogram's cost), and bins laid over
+  // [floor, max] instead of the keys' common prefix hold fewer each to rank
+  // (decode at 32K keys 64.7 -> 63.0 us per step, one row 23.1 -> 21.8).
   int nv = 0;
-  unsigned kmin = 0xffffffffu, kmax = 0u;
+  unsigned kmin = 0xffffffffu, kmax = 0u, k2 = 0u;
 #pragma unroll
-  for (int u = 0; u < kFastKpt; ++u) {
+  for (int u = 0; u < KPT; ++u) {
     const bool v = kr[u] > kNegInfKey;
     nv += v;
     kmin = v ? min(kmin, kr[u]) : kmin;
-    kmax = v ? max(kmax, kr[u]) : kmax;
+    k2 = max(k2, min(kmax, kr[u]));  // second largest
+    kmax = max(kmax, kr[u]);
   }
   {
+    const unsigned tt = K <= kTopkThreads ? kmax : K <= 2 * kTopkThreads ? k2 : 0u;
     const unsigned tn = wave_reduce_to63((unsigned)nv, 0u, [](unsigned a, unsigned b) { return a + b; });
     const unsigned tmin = wave_reduce_to63(kmin, 0xffffffffu, [](unsigned a, unsigned b) { return min(a, b); });
     const unsigned tmax = wave_reduce_to63(kmax, 0u, [](unsigned a, unsigned b) { return max(a, b); });
+    const unsigned tflo = wave_reduce_to63(tt, 0xffffffffu, [](unsigned a, unsigned b) { return min(a, b); });
     if (lane == 63) {
       misc[wave] = tn;
       misc[kTopkWaves + wave] = tmin;
       misc[2 * kTopkWaves + wave] = tmax;
+      wsum[wave] = tflo;
     }
+    if (tid == 0) *s_big = 0u;
   }
   __syncthreads();
   int n_valid = 0;
-  kmin = 0xffffffffu;
+  unsigned lo = 0xffffffffu, flo = 0xffffffffu;
   kmax = 0u;
 #pragma unroll
   for (int w = 0; w < kTopkWaves; ++w) {
     n_valid += (int)misc[w];
-    kmin = min(kmin, misc[kTopkWaves + w]);
+    lo = min(lo, misc[kTopkWaves + w]);
     kmax = max(kmax, misc[2 * kTopkWaves + w]);
+    flo = min(flo, wsum[w]);
   }
+  lo = max(lo, flo);
   const int take = min(K, n_valid);
-  const unsigned diff = kmin ^ kmax;
-  const int hb = diff ? 32 - __clz((int)diff) : 0;
+  const unsigned diff = kmax - lo;
+  const int hb = n_valid > 0 && diff ? 32 - __clz((int)diff) : 0;
   const int shift = hb > 12 ? hb - 12 : 0;
-  auto digit = [&](unsigned kk) { return (kk >> shift) & (unsigned)(kFastBins - 1); };
+  auto digit = [&](unsigned kk) { return (kk - lo) >> shift; };  // keys from lo up
 
   // ---- 2. histogram, bin starts (descending), threshold bin ----
   if (take > 0) {
 #pragma unroll
-    for (int u = 0; u < kFastKpt; ++u)
-      if (kr[u] > kNegInfKey) atomicAdd(&hcount[digit(kr[u])], 1u);
+    for (int u = 0; u < KPT; ++u)
+      if (kr[u] >= lo) atomicAdd(&hcount[digit(kr[u])], 1u);
   }
   __syncthreads();  // also: misc reads done before misc is rewritten
   int ncand = 0;
   unsigned bstar = 0;
   if (take > 0) {
     // thread t owns bins 4095 - 4t - i (descending), i = 0..3
-    unsigned c[4], ex[4];
-#pragma unroll
-    for (int i = 0; i < 4; ++i) ex[i] = c[i] = hcount[kFastBins - 1 - 4 * tid - i];
+    const u32x4 hv = *(const u32x4*)&hcount[kFastBins - 4 - 4 * tid];
+    const unsigned c[4] = {hv[3], hv[2], hv[1], hv[0]};
+    unsigned ex[4] = {c[0], c[1], c[2], c[3]};
     block_scan4(ex, wsum);
+    const u32x4 bv = {ex[3], ex[2], ex[1], ex[0]};
+    *(u32x4*)&hbase[kFastBins - 4 - 4 * tid] = bv;
+    *(u32x4*)&cursor[kFastBins - 4 - 4 * tid] = bv;
+    // the candidates' bins are those that start before slot `take`
+    unsigned cm = 0;
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
-      const int b = kFastBins - 1 - 4 * tid - i;
-      hbase[b] = ex[i];
-      cursor[b] = ex[i];
+      if (ex[i] < (unsigned)take) cm = max(cm, c[i]);
       if (ex[i] < (unsigned)take && ex[i] + c[i] >= (unsigned)take) {
-        misc[0] = (unsigned)b;    // b*
-        misc[1] = ex[i] + c[i];   // keys in bins >= b*
+        misc[0] = (unsigned)(kFastBins - 1 - 4 * tid - i);  // b*
+        misc[1] = ex[i] + c[i];                             // keys in bins >= b*
       }
     }
-    if (tid == 0) misc[2] = 0u;
+    cm = wave_reduce_to63(cm, 0u, [](unsigned a, unsigned b) { return max(a, b); });
+    if (lane == 63 && cm) atomicMax(s_big, cm);
     __syncthreads();
     bstar = misc[0];
     ncand = (int)misc[1];
-    // largest bin among the candidates' bins
-    unsigned cm = 0;
-#pragma unroll
-    for (int i = 0; i < 4; ++i) cm = (unsigned)(kFastBins - 1 - 4 * tid - i) >= bstar ? max(cm, c[i]) : cm;
-    cm = wave_reduce_to63(cm, 0u, [](unsigned a, unsigned b) { return max(a, b); });
-    if (lane == 63 && cm) atomicMax(&misc[2], cm);
-    __syncthreads();
-    if (ncand > kFastCap || misc[2] > (unsigned)kSegCap) {
+    if (ncand > kFastCap || *s_big > (unsigned)kSegCap) {
       // crowded keys: the general selection (uniform branch)
       __syncthreads();
       topk_row_generic<IN_LDS>(p, row, tk_smem);
@@ -1442,11 +1454,11 @@ __global__ __launch_bounds__(kTopkThreads) void li_topk_kernel(TopkParams p) {
     // ---- 3. counting sort of the candidates by bin ----
     // each candidate takes a slot of its bin's range in cand from the bin's
     // cursor (the order inside a bin is arbitrary: step 4 ranks by key)
+    const unsigned cut = lo + (bstar << shift);  // the smallest key of bin b*
 #pragma unroll
-    for (int u = 0; u < kFastKpt; ++u) {
-      const unsigned d = digit(kr[u]);
-      if (kr[u] > kNegInfKey && d >= bstar) {
-        const unsigned slot = atomicAdd(&cursor[d], 1u);
+    for (int u = 0; u < KPT; ++u) {
+      if (kr[u] >= cut) {
+        const unsigned slot = atomicAdd(&cursor[digit(kr[u])], 1u);
         cand[slot] = ((unsigned long long)(~kr[u]) << 32) | (unsigned)entry(u);
       }
     }
@@ -1878,13 +1890,14 @@ int li_topk_run(const float* scores, int64_t rows, int64_t s2, int64_t k, int32_
   const bool in_lds = li_topk_row_in_lds(s2, k);
   size_t lds = li_topk_fixed_bytes(k) + (in_lds ? (size_t)s2 * 4 : 0);  // general path
   if (lds < kFastLds) lds = kFastLds;
-  const void* fn = in_lds ? (const void*)li_topk_kernel<true> : (const void*)li_topk_kernel<false>;
+  const void* fn;
+  if (s2 <= 8 * kTopkThreads) fn = in_lds ? (const void*)li_topk_kernel<true, 8> : (const void*)li_topk_kernel<false, 8>;
+  else if (s2 <= 16 * kTopkThreads) fn = in_lds ? (const void*)li_topk_kernel<true, 16> : (const void*)li_topk_kernel<false, 16>;
+  else if (s2 <= 24 * kTopkThreads) fn = in_lds ? (const void*)li_topk_kernel<true, 24> : (const void*)li_topk_kernel<false, 24>;
+  else fn = in_lds ? (const void*)li_topk_kernel<true, 32> : (const void*)li_topk_kernel<false, 32>;
   DSA_HIP(hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, kTopkLdsBudget));
-  if (in_lds)
-    hipLaunchKernelGGL(li_topk_kernel<true>, dim3((unsigned)rows), dim3(kTopkThreads), lds, stream, p);
-  else
-    hipLaunchKernelGGL(li_topk_kernel<false>, dim3((unsigned)rows), dim3(kTopkThreads), lds, stream, p);
-  DSA_HIP(hipGetLastError());
+  void* args[] = {&p};
+  DSA_HIP(hipLaunchKernel(fn, dim3((unsigned)rows), dim3(kTopkThreads), args, lds, stream));
   return DSA_OK;
 }
 
