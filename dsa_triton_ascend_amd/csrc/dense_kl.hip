@@ -281,7 +281,7 @@ __global__ __launch_bounds__(256, NHT > 4 ? 2 : 3) void dense_index_rows_kernel(
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int li = lane & 15, lg = lane >> 4;
-  const int groups = (p.s1 + 3) / 4;
+  const int groups = p.s1 / 4 + (p.s1 % 4 != 0);
   const int b = blockIdx.x % p.batch;
   const int s0 = (groups - 1 - (int)(blockIdx.x / p.batch)) * 4;  // long causal rows first
   const int aq = p.act_q ? p.act_q[b] : p.s1;
@@ -975,7 +975,7 @@ __global__ __launch_bounds__(256, 2) void dense_dqi_tile_kernel(DkParams p) {
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int li = lane & 15, lg = lane >> 4;
   const int hgr = p.nidx / kDkCols, rpw = 4 / hgr;  // head groups per row, rows per workgroup
-  const int groups = (p.s1 + rpw - 1) / rpw;
+  const int groups = p.s1 / rpw + (p.s1 % rpw != 0);
   const int b = blockIdx.x % p.batch;
   const int s0 = (groups - 1 - (int)(blockIdx.x / p.batch)) * rpw;  // long causal rows first
   const int s1 = s0 + wave / hgr, g0 = (wave % hgr) * kDkCols;
@@ -1242,7 +1242,9 @@ static int dk_chunk(int64_t batch, int64_t s1, int64_t s2) {
   const int64_t full = s2 >= s1 ? std::min(n, (s2 - s1) / kDkKeys + 1) : 0;
   const int64_t total = full * s1 + (n - full) * s2 - kDkKeys * ((n * (n - 1) - full * (full - 1)) / 2);
   const int64_t cus = device_cu_count(), wgs = std::max(cus, 2 * cus - batch * n);
-  return (int)std::min<int64_t>(1 << 20, std::max<int64_t>(32, (batch * total + wgs - 1) / wgs));
+  // (at most 64 chunks of a key tile, which bounds the partials' workspace)
+  const int64_t even = std::max((batch * total + wgs - 1) / wgs, (s1 + 63) / 64);
+  return (int)std::max<int64_t>(32, std::min<int64_t>(even, 1 << 23));
 }
 static int64_t dk_part_splits(int64_t batch, int64_t s1, int64_t s2, int64_t di) {
   const int64_t sp = dense_kl_splits(batch, s1, s2);
@@ -1283,7 +1285,7 @@ template <typename T>
 static hipError_t dk_index(const DkParams& p, int di, hipStream_t stream) {
   const dim3 grid((unsigned)(p.batch * p.s1));
   if (di == kDkRowDi) {
-    const dim3 g4((unsigned)(p.batch * ((p.s1 + 3) / 4)));
+    const dim3 g4((unsigned)(p.batch * (((int64_t)p.s1 + 3) / 4)));
     if (p.nidx <= 32) hipLaunchKernelGGL((dense_index_rows_kernel<2, T>), g4, dim3(256), 0, stream, p);
     else if (p.nidx <= 64) hipLaunchKernelGGL((dense_index_rows_kernel<4, T>), g4, dim3(256), 0, stream, p);
     else hipLaunchKernelGGL((dense_index_rows_kernel<8, T>), g4, dim3(256), 0, stream, p);
@@ -1314,9 +1316,9 @@ static hipError_t dk_grads(const DkParams& p, int di, void* d_key_index, hipStre
   const dim3 kgrid((unsigned)(p.batch * ntiles * p.splits));
   if (dk_tiles(p.nidx, di)) {
     const int rpw = 4 / (p.nidx / kDkCols);
-    hipLaunchKernelGGL((dense_dqi_tile_kernel<T>), dim3((unsigned)(p.batch * ((p.s1 + rpw - 1) / rpw))), dim3(256), 0,
+    hipLaunchKernelGGL((dense_dqi_tile_kernel<T>), dim3((unsigned)(p.batch * (((int64_t)p.s1 + rpw - 1) / rpw))), dim3(256), 0,
                        stream, p);
-    const int64_t chunks = (p.s1 + p.chunk - 1) / p.chunk;
+    const int64_t chunks = ((int64_t)p.s1 + p.chunk - 1) / p.chunk;
     hipLaunchKernelGGL((dense_dki_tile_kernel<T>), dim3((unsigned)((p.batch * ntiles + 7) / 8 * 8 * chunks)), dim3(256), 0, stream, p);
     const int64_t n4t = (int64_t)p.batch * p.s2 * di / 4;
     hipLaunchKernelGGL((dense_dki_tile_reduce_kernel<T>), dim3((unsigned)((n4t + 255) / 256)), dim3(256), 0, stream, p,
