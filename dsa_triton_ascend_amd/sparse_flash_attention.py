@@ -70,6 +70,8 @@ def _expect_numel(t, n, name):
 def _band_args(pre_tokens, next_tokens):
     """pre_tokens / next_tokens as Python ints in int64 range (the C-ABI
     takes int64_t; ctypes would wrap larger values silently)."""
+    if type(pre_tokens) is int and type(next_tokens) is int and pre_tokens == next_tokens == INT64_MAX:
+        return pre_tokens, next_tokens
     out = []
     for name, v in (("pre_tokens", pre_tokens), ("next_tokens", next_tokens)):
         if isinstance(v, torch.Tensor):
@@ -197,9 +199,11 @@ def sparse_flash_attention_triton(
         raise ValueError(f"N1 must be one of {_VALID_N1}, got {N1}")
     if query.dtype not in (torch.bfloat16, torch.float16):
         raise ValueError(f"query dtype must be bfloat16 or float16, got {query.dtype}")
-    for name, t in (("key", key), ("query_rope", query_rope), ("key_rope", key_rope)):
-        if t.dtype != query.dtype:
-            raise ValueError(f"{name} dtype {t.dtype} differs from query dtype {query.dtype}")
+    dtype = query.dtype
+    if key.dtype != dtype or query_rope.dtype != dtype or key_rope.dtype != dtype:
+        for name, t in (("key", key), ("query_rope", query_rope), ("key_rope", key_rope)):
+            if t.dtype != dtype:
+                raise ValueError(f"{name} dtype {t.dtype} differs from query dtype {dtype}")
     if (act_k is not None and act_k.numel() != B) or (act_q is not None and act_q.numel() != B):
         raise ValueError("actual sequence length arrays must have one entry per batch")
 
@@ -210,8 +214,11 @@ def sparse_flash_attention_triton(
     if key.dim() != (3 if is_tnd_kv else 4) or key.shape[-1] != D:
         raise ValueError(f"key must be {'[T2,1,D]' if is_tnd_kv else '[B,S2,1,D]'} with D={D}, "
                          f"got {tuple(key.shape)}")
-    _expect_shape(query_rope, tuple(query.shape[:-1]) + (D_ROPE,), "query_rope")
-    _expect_shape(key_rope, tuple(key.shape[:-1]) + (D_ROPE,), "key_rope")
+    # compared without building the expected shapes (the smallest calls are bound by this function's own time)
+    if query_rope.shape[:-1] != query.shape[:-1]:
+        _expect_shape(query_rope, tuple(query.shape[:-1]) + (D_ROPE,), "query_rope")
+    if key_rope.shape[-1] != D_ROPE or key_rope.shape[:-1] != key.shape[:-1]:
+        _expect_shape(key_rope, tuple(key.shape[:-1]) + (D_ROPE,), "key_rope")
     if is_pa and (bt.dim() != 2 or bt.shape[0] < B):
         raise ValueError(f"block_table must be [B, max_blocks] with B={B} rows, got {tuple(bt.shape)}")
     _check_device(query, key, query_rope, key_rope, sparse_indices, block_table)
@@ -220,15 +227,15 @@ def sparse_flash_attention_triton(
     qr = query_rope.contiguous()
     k = key.contiguous()
     kr = key_rope.contiguous()
-    si = sparse_indices.to(dtype=torch.int32).contiguous()
+    si = sparse_indices if sparse_indices.dtype is torch.int32 else sparse_indices.to(dtype=torch.int32)
+    si = si.contiguous()
 
-    out_shape = (q_rows, N1, D) if is_tnd_q else (B, S1, N1, D)
     lse_shape = (1, q_rows, N1) if is_tnd_q else (B, 1, S1, N1)
-    out = torch.empty(out_shape, dtype=query.dtype, device=device)
+    out = torch.empty_like(q, memory_format=torch.contiguous_format)
     # the library writes the statistics, or zeros when they are not
     # requested (no fill kernels of torch's own per call)
     smax = torch.empty(lse_shape, dtype=torch.float32, device=device)
-    ssum = torch.empty(lse_shape, dtype=torch.float32, device=device)
+    ssum = torch.empty_like(smax)
     if q_rows == 0:
         return out, smax, ssum
 
@@ -236,13 +243,13 @@ def sparse_flash_attention_triton(
     ws_bytes = lib.dsa_sfa_fwd_workspace_size(q_rows, N1, D, K, sparse_block_size)
     ws = torch.empty(max(ws_bytes, 1), dtype=torch.uint8, device=device) if ws_bytes else None
     status = lib.dsa_sfa_fwd(
-        _lib.ptr(q), _lib.ptr(qr), _lib.ptr(k), _lib.ptr(kr), _lib.ptr(si),
-        _lib.ptr(out), _lib.ptr(smax), _lib.ptr(ssum),
+        q.data_ptr(), qr.data_ptr(), k.data_ptr(), kr.data_ptr(), si.data_ptr(),
+        out.data_ptr(), smax.data_ptr(), ssum.data_ptr(),
         _lib.ptr(act_q), _lib.ptr(act_k), _lib.ptr(bt),
         B, S1, S2, N1, D, D_ROPE, K, q_rows, kv_rows, max_blocks, page,
         sparse_block_size, sparse_mode, pre_tokens, next_tokens, _lib.LAYOUT[layout_query],
         _lib.LAYOUT[layout_kv],
-        _lib.dtype_code(query.dtype), float(scale_value), 1 if return_softmax_lse else 0,
+        _lib.dtype_code(dtype), float(scale_value), 1 if return_softmax_lse else 0,
         _lib.ptr(ws), ws_bytes, _lib.stream_handle(device))
     _lib.check(status, "dsa_sfa_fwd")
     return out, smax, ssum
