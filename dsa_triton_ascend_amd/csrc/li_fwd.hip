@@ -22,10 +22,9 @@
 //
 // Top-k kernel: one workgroup (1024 threads) per row.  Scores map to
 // order-preserving uint32 keys.  Rows of up to 32768 scores take the fast
-// selection (li_topk_kernel below): a 4096-bin histogram of the 12 key bits
-// under the common prefix of the row's finite keys finds the bin holding
-// the K-th largest key; the candidates in that bin and above are counting-
-// sorted by bin, and each one's final position is its bin start plus its
+// selection (li_topk_kernel below): a 4096-bin histogram of the keys above a
+// floor under the answer finds the bin holding the K-th largest key; the
+// candidates in that bin and above are counting-sorted by bin, and each one's final position is its bin start plus its
 // rank within the bin by the composite (~key << 32 | index), which is
 // exactly score descending / index ascending.  Wider rows, more than 4096
 // candidates, or a crowded bin take the general selection: a radix select
