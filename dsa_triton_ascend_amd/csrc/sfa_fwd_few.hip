@@ -362,7 +362,9 @@ __global__ __launch_bounds__(TW * 64, 1) void sfa_fwd_few_kernel(SfaFwdParams p)
           n_total += __popcll(m);
         }
       }
-      if (last && lane < TILE) list[n_list + lane] = -1;
+      // pad to a whole tile; with entries left over from earlier chunks the list
+      // can be full to its last entry, and the pad ends there
+      if (last && lane < TILE && n_list + lane < LIST) list[n_list + lane] = -1;
       wave_lds_sync();
       if (!last) load_ids(c + kFewChunk);
       const int nt = last ? (n_list + TILE - 1) / TILE : n_list / TILE;

@@ -21,7 +21,7 @@ pytestmark = pytest.mark.gpu
 D = 512
 
 
-def _check(S1, S2, N1, K, mode, dtype, bs=1, mul=1.0, flags=0, act_k=None, punch=False, seed=5):
+def _check(S1, S2, N1, K, mode, dtype, bs=1, mul=1.0, flags=0, act_k=None, punch=False, holes=(), seed=5):
     import dsa_triton_ascend_amd as dsa
     from dsa_triton_ascend_amd import _lib
     print(f"[few heads] S1={S1} S2={S2} N1={N1} K={K} mode={mode} bs={bs} {dtype} x{mul} flags={flags}", flush=True)
@@ -32,6 +32,8 @@ def _check(S1, S2, N1, K, mode, dtype, bs=1, mul=1.0, flags=0, act_k=None, punch
         rng = np.random.RandomState(3)
         si[rng.rand(*si.shape) < 0.4] = -1
         si[:, ::7] = -1
+    for h in holes:
+        si[..., h] = -1
     scale = 1.0 / np.sqrt(D + 64)
     lib = _lib.load()
     if flags:
@@ -65,6 +67,15 @@ def test_rows_and_lengths(S1, K, N1, dtype):
 @pytest.mark.parametrize("N1", [16, 32])
 def test_holes_short_rows_and_causal_start(S1, N1):
     _check(S1, S1, N1, 600, 3, torch.bfloat16, punch=True)
+
+
+@pytest.mark.parametrize("S1,K,holes", [(800, 1024, (0,)), (130, 4096, (0, 1024, 2048, 3072))])
+@pytest.mark.parametrize("N1", [16, 32])
+def test_list_full_to_its_last_entry(S1, K, holes, N1):
+    """One hole in a wave's first 512 positions leaves 15 entries for the next
+    chunk, whose 512 then fill the list: the pad must stay inside it (the next
+    wave's list follows)."""
+    _check(S1, K + 100, N1, K, 0, torch.bfloat16, holes=holes)
 
 
 @pytest.mark.parametrize("S1", [130, 800])
