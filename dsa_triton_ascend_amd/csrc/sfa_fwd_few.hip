@@ -23,9 +23,12 @@
 //  * At 32 heads O^T += V^T . P^T runs on 32x32x16: the C layout of S^T becomes
 //    its B layout by two v_permlane16_swap of the packed numerators (no LDS);
 //    at 16 heads on 16x16x16, whose B layout is the C layout of S^T.
-//  * The reference max of a head is its first tile's; scores that pass it by
+//  * The reference max of a head is that of the row's first 32 tokens (two
+//    tiles, scored once before the loop), as in sfa_fwd.hip, and one for all
+//    waves of a row: the numerators round as they do there, and a large score
+//    at the start of a row is every wave's reference.  Scores that pass it by
 //    more than kRefSlack (log2 units) send the wave through its positions a
-//    second time with the exact maxima, as in sfa_fwd.hip.
+//    second time with the exact maxima.
 //  * TW = 1 (many rows: prefill): one wave per workgroup and row, four
 //    workgroups per CU.  TW = 4 (fewer rows than wave slots): a row's positions
 //    are dealt to four waves, whose (O, max, sum) are merged in fp32 through
@@ -80,7 +83,8 @@ __global__ __launch_bounds__(TW * 64, 1) void sfa_fwd_few_kernel(SfaFwdParams p)
   __shared__ __attribute__((aligned(1024))) unsigned char smem[TW][2 * BUFB];
   __shared__ int s_list[TW][LIST];
   __shared__ float s_st[TW > 1 ? TW : 1][3][HEADS];
-  __shared__ int s_cnt[TW];
+  __shared__ float s_ref[HEADS];
+  __shared__ int s_cnt[TW], s_tiles[TW];
 
   const int tid = threadIdx.x;
   const int lane = tid & 63;
@@ -215,15 +219,14 @@ __global__ __launch_bounds__(TW * 64, 1) void sfa_fwd_few_kernel(SfaFwdParams p)
   // use until the end of tile t - 1's second product), GEMM2 the rope rows and
   // the first three quarters of tile t + 2, each into a quarter of tile t's
   // buffer whose columns are done.
-  auto run_tile = [&](int b, int nleft, bool with_lo, bool dma1, const Rows& r1, bool dma2, const Rows& r2) {
+  auto gemm1 = [&](int b, f32x4 (&s)[HT][2], bool dma1, const Rows& r1) {
     const unsigned char* buf = ring + b * BUFB;
-    int g1 = g1_lane, g2 = g2_lane, g2b = g2b_lane;
-    asm volatile("" : "+v"(g1), "+v"(g2), "+v"(g2b));  // the offsets below are not held across tiles
+    int g1 = g1_lane;
+    asm volatile("" : "+v"(g1));  // the offsets below are not held across tiles
     auto kfrag = [&](int ks) -> V8 {
       if (ks < KSN) return as_v8<V8>(*(const u32x4*)(buf + (g1 ^ ((ks & 3) << 6)) + (ks >> 2) * 4096));
       return as_v8<V8>(*(const u32x4*)(buf + (g1r ^ ((ks - KSN) << 6))));
     };
-    f32x4 s[HT][2];
 #pragma unroll
     for (int ht = 0; ht < HT; ++ht) s[ht][0] = s[ht][1] = (f32x4){0.f, 0.f, 0.f, 0.f};
     constexpr int PF = 6;  // K fragments in flight
@@ -239,6 +242,23 @@ __global__ __launch_bounds__(TW * 64, 1) void sfa_fwd_few_kernel(SfaFwdParams p)
       if (ks < 4 && dma1) issue_nope(r1, b ^ 1, 3, ks);
       __builtin_amdgcn_sched_barrier(0);
     }
+  };
+  // scores of head tile ht in log2 units, lane -> head li, tokens 4 lg + r; returns their max
+  auto scaled = [&](const f32x4 (&s)[HT][2], int ht, int nleft, float (&v)[4]) -> float {
+    float tmax = -INFINITY;
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      v[r] = lg * 4 + r < nleft ? (s[ht][0][r] + s[ht][1][r]) * p.scale_log2 : -INFINITY;
+      tmax = fmaxf(tmax, v[r]);
+    }
+    return xgroup_max(tmax);
+  };
+  auto run_tile = [&](int b, int nleft, bool with_lo, bool dma1, const Rows& r1, bool dma2, const Rows& r2) {
+    const unsigned char* buf = ring + b * BUFB;
+    f32x4 s[HT][2];
+    gemm1(b, s, dma1, r1);
+    int g2 = g2_lane, g2b = g2b_lane;
+    asm volatile("" : "+v"(g2), "+v"(g2b));  // the offsets below are not held across tiles
     // the first V^T fragments are on their way during the softmax
     constexpr int PV = 4;
     typedef std::conditional_t<HT == 2, i16x8, s16x4> VFrag;
@@ -258,13 +278,8 @@ __global__ __launch_bounds__(TW * 64, 1) void sfa_fwd_few_kernel(SfaFwdParams p)
     T4 hi[HT], lo[HT];
 #pragma unroll
     for (int ht = 0; ht < HT; ++ht) {
-      float v[4], tmax = -INFINITY;
-#pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        v[r] = lg * 4 + r < nleft ? (s[ht][0][r] + s[ht][1][r]) * p.scale_log2 : -INFINITY;
-        tmax = fmaxf(tmax, v[r]);
-      }
-      tmax = xgroup_max(tmax);
+      float v[4];
+      const float tmax = scaled(s, ht, nleft, v);
       m_true[ht] = fmaxf(m_true[ht], tmax);
       if (!exact_ref && m_ref[ht] == -INFINITY) m_ref[ht] = tmax;
       overflow |= tmax > m_ref[ht] + kRefSlack;
@@ -326,84 +341,134 @@ __global__ __launch_bounds__(TW * 64, 1) void sfa_fwd_few_kernel(SfaFwdParams p)
   };
 
   // ---- chunks of positions: compact, then run the whole tiles; what is left
-  // of a chunk (fewer than TILE tokens) opens the next one's list.  A head
-  // whose scores pass the reference max by more than the slack sends the wave
-  // through its positions once more, with the exact maxima as references.
+  // of a chunk (fewer than TILE tokens) opens the next one's list.
   const int32_t* gtab = p.layout_kv == DSA_LAYOUT_PA_BSND ? p.block_table + (int64_t)ri.b * p.max_blocks : nullptr;
+  int n_list = 0, n_total = 0, nt = 0;
+  Rows r1 = {};
+  // the list of chunk c, its whole tiles nt, and the first two on their way
+  // (without the last quarter of the second: r1)
+  auto open_chunk = [&](int c, bool last) {
+    {
+      int phys[RPL];
+      unsigned ok = 0;
+#pragma unroll
+      for (int u = 0; u < RPL; ++u) {
+        phys[u] = 0;
+        const int pos = c + u * 64 + lane;
+        const bool v = ri.active && pos < p1 && sfa_resolve_id(p, ri, ids[u], pos, &phys[u], gtab);
+        ok |= (unsigned)v << u;
+      }
+#pragma unroll
+      for (int u = 0; u < RPL; ++u) {
+        const bool v = (ok >> u) & 1;
+        const unsigned long long m = __ballot(v);
+        if (v) list[n_list + __popcll(m & ((1ull << lane) - 1ull))] = phys[u];
+        n_list += __popcll(m);
+        n_total += __popcll(m);
+      }
+    }
+    // pad to a whole tile; with entries left over from earlier chunks the list
+    // can be full to its last entry, and the pad ends there
+    if (last && lane < TILE && n_list + lane < LIST) list[n_list + lane] = -1;
+    wave_lds_sync();
+    if (!last) load_ids(c + kFewChunk);
+    nt = last ? (n_list + TILE - 1) / TILE : n_list / TILE;
+    if (nt > 0) {
+      const Rows r0 = rows_of(0);
+#pragma unroll
+      for (int j = 0; j < 2; ++j) issue_rope(r0, 0, j);
+#pragma unroll
+      for (int q = 0; q < 4; ++q)
+#pragma unroll
+        for (int j = 0; j < 4; ++j) issue_nope(r0, 0, q, j);
+    }
+    if (nt > 1) {
+      r1 = rows_of(1);
+#pragma unroll
+      for (int j = 0; j < 2; ++j) issue_rope(r1, 1, j);
+#pragma unroll
+      for (int q = 0; q < 3; ++q)
+#pragma unroll
+        for (int j = 0; j < 4; ++j) issue_nope(r1, 1, q, j);
+    }
+  };
+
+  // ---- the reference maxima, from the row's first two tiles: the first wave
+  // with a tile in its first chunk scores them for all.  (Before the
+  // accumulators are in use: beside them a second copy of the product made
+  // the 32-head kernels spill.)
   int n_others = 0;  // tokens of the other waves' first chunks
-  if (TW > 1 && kSplitP && p0 >= p1) {
-    if (lane == 0) s_cnt[wave] = 0;
+  const bool last0 = p0 + kFewChunk >= p1;
+  bool primed = false;  // tile 1 is on its way whole
+  if (p0 < p1) open_chunk(p0, last0);
+  bool first = nt > 0;
+  if constexpr (TW > 1) {
+    if (lane == 0) {
+      s_cnt[wave] = n_total;
+      s_tiles[wave] = nt;
+    }
     lds_barrier();
+#pragma unroll
+    for (int w = 0; w < TW; ++w) {
+      n_others += w == wave ? 0 : s_cnt[w];
+      first = first && (w >= wave || s_tiles[w] == 0);
+    }
   }
+  if (first) {
+    primed = nt > 1;
+    if (primed) {
+#pragma unroll
+      for (int j = 0; j < 4; ++j) issue_nope(r1, 1, 3, j);
+    }
+#pragma unroll 1
+    for (int t = 0; t < min(nt, 2); ++t) {
+      if (t == 0 && primed) wait_vmcnt<NDMA>();  // tile 1's
+      else wait_vmcnt<0>();
+      f32x4 s[HT][2];
+      gemm1(t, s, false, r1);
+#pragma unroll
+      for (int ht = 0; ht < HT; ++ht) {
+        float v[4];
+        m_ref[ht] = fmaxf(m_ref[ht], scaled(s, ht, n_list - t * TILE, v));
+      }
+    }
+  }
+  if constexpr (TW > 1) {
+    if (first && lg == 0) {
+#pragma unroll
+      for (int ht = 0; ht < HT; ++ht) s_ref[ht * 16 + li] = m_ref[ht];
+    }
+    lds_barrier();
+    bool any = false;
+#pragma unroll
+    for (int w = 0; w < TW; ++w) any = any || s_tiles[w] > 0;
+#pragma unroll
+    for (int ht = 0; ht < HT; ++ht) m_ref[ht] = any ? s_ref[ht * 16 + li] : -INFINITY;
+  }
+
+  // A head whose scores pass the reference max by more than the slack sends
+  // the wave through its positions once more, with the exact maxima as
+  // references.
   for (int pass = 0; pass < 2; ++pass) {
 #pragma unroll
     for (int d = 0; d < NDT; ++d)
 #pragma unroll
       for (int r = 0; r < NACC; ++r) acc[d][r] = 0.f;
-    int n_list = 0, n_total = 0;
     for (int c = p0; c < p1; c += kFewChunk) {
       const bool last = c + kFewChunk >= p1;
-      {
-        int phys[RPL];
-        unsigned ok = 0;
-#pragma unroll
-        for (int u = 0; u < RPL; ++u) {
-          phys[u] = 0;
-          const int pos = c + u * 64 + lane;
-          const bool v = ri.active && pos < p1 && sfa_resolve_id(p, ri, ids[u], pos, &phys[u], gtab);
-          ok |= (unsigned)v << u;
-        }
-#pragma unroll
-        for (int u = 0; u < RPL; ++u) {
-          const bool v = (ok >> u) & 1;
-          const unsigned long long m = __ballot(v);
-          if (v) list[n_list + __popcll(m & ((1ull << lane) - 1ull))] = phys[u];
-          n_list += __popcll(m);
-          n_total += __popcll(m);
-        }
-      }
-      // pad to a whole tile; with entries left over from earlier chunks the list
-      // can be full to its last entry, and the pad ends there
-      if (last && lane < TILE && n_list + lane < LIST) list[n_list + lane] = -1;
-      wave_lds_sync();
-      if (!last) load_ids(c + kFewChunk);
-      const int nt = last ? (n_list + TILE - 1) / TILE : n_list / TILE;
-      // the lo part of P: while the workgroup has seen fewer tokens than the
-      // rule says (a wave without positions counts none, below)
-      if (TW > 1 && kSplitP && pass == 0 && c == p0) {
-        if (lane == 0) s_cnt[wave] = n_total;
-        lds_barrier();
-        n_others = 0;
-#pragma unroll
-        for (int w = 0; w < TW; ++w) n_others += w == wave ? 0 : s_cnt[w];
-      }
+      if (pass > 0 || c > p0) open_chunk(c, last);
+      // the lo part of P: while the workgroup has seen fewer tokens than the rule says
       const bool with_lo = n_total + n_others < kLoSplitMinTokens || pass > 0;
-      Rows r1 = {}, r2 = {};
-      if (nt > 0) {
-        const Rows r0 = rows_of(0);
-#pragma unroll
-        for (int j = 0; j < 2; ++j) issue_rope(r0, 0, j);
-#pragma unroll
-        for (int q = 0; q < 4; ++q)
-#pragma unroll
-          for (int j = 0; j < 4; ++j) issue_nope(r0, 0, q, j);
-      }
-      if (nt > 1) {
-        r1 = rows_of(1);
-#pragma unroll
-        for (int j = 0; j < 2; ++j) issue_rope(r1, 1, j);
-#pragma unroll
-        for (int q = 0; q < 3; ++q)
-#pragma unroll
-          for (int j = 0; j < 4; ++j) issue_nope(r1, 1, q, j);
-      }
+      Rows r2 = {};
+#pragma unroll 1  // (nor peeled for `primed`: a second copy of the loop body spills)
       for (int t = 0; t < nt; ++t) {
         // all of tile t is in; 14 DMAs of tile t + 1 came after it (a later
         // load of the compiler's own only makes this wait longer)
         if (t + 1 < nt) wait_vmcnt<NDMA - 4>();
         else wait_vmcnt<0>();
         if (t + 2 < nt) r2 = rows_of(t + 2);
-        run_tile(t & 1, n_list - t * TILE, with_lo, t + 1 < nt, r1, t + 2 < nt, r2);
+        run_tile(t & 1, n_list - t * TILE, with_lo, t + 1 < nt && !primed, r1, t + 2 < nt, r2);
+        primed = false;
         r1 = r2;
       }
       if (!last) {
@@ -421,6 +486,7 @@ __global__ __launch_bounds__(TW * 64, 1) void sfa_fwd_few_kernel(SfaFwdParams p)
       m_ref[ht] = m_true[ht];
       l_run[ht] = 0.f;
     }
+    n_list = n_total = 0;
     load_ids(p0);
   }
 

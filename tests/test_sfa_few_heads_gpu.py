@@ -115,3 +115,70 @@ def test_paged_equals_dense(B, S1, N1):
                                           actual_seq_lengths_kv=[S2] * B, **kw)
     for x, y in zip(a, b):
         assert torch.equal(x, y)
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16], ids=["bf16", "fp16"])
+@pytest.mark.parametrize("N1", [16, 32])
+@pytest.mark.parametrize("S1", [130, 800])
+def test_numerators_round_as_on_the_wide_kernel(S1, N1, dtype):
+    """The softmax numerators are rounded relative to the same reference as on
+    the 128-head kernels (the max of the row's first 32 tokens), so the outputs
+    agree but for the order of the fp32 sums.  Those leave the scores (|s| < 16
+    log2 units) and sums within about 1e-6 of each other: at most some 1 % of
+    the numerators and outputs land on another 16-bit value.  With another
+    reference every numerator rounds anew, and a quarter of the outputs differ."""
+    import dsa_triton_ascend_amd as dsa
+    from dsa_triton_ascend_amd import _lib
+    print(f"[few heads] wide kernel S1={S1} N1={N1} {dtype}", flush=True)
+    K = 1024
+    q, k, qr, kr = sfa_inputs(1, S1, 1500, N1, D, dtype)
+    si = sparse_indices(1, S1, 1500, K, 1, 0)
+    args = (dev(q, dtype), dev(k, dtype), None, dev(si, torch.int32))
+    kw = dict(scale_value=1.0 / np.sqrt(D + 64), query_rope=dev(qr, dtype), key_rope=dev(kr, dtype), sparse_mode=0,
+              return_softmax_lse=True)
+    a = dsa.sparse_flash_attention_triton(*args, **kw)
+    lib = _lib.load()
+    lib.dsa_set_test_flags(8)
+    try:
+        b = dsa.sparse_flash_attention_triton(*args, **kw)
+        torch.cuda.synchronize()
+    finally:
+        lib.dsa_set_test_flags(0)
+    differ = (a[0] != b[0]).float().mean().item()
+    print(f"[few heads] {differ:.2g} of the outputs differ", flush=True)
+    assert differ < 0.08
+    torch.testing.assert_close(a[1], b[1], rtol=1e-6, atol=1e-6)
+    torch.testing.assert_close(a[2], b[2], rtol=1e-5, atol=0)
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16], ids=["bf16", "fp16"])
+@pytest.mark.parametrize("S1", [130, 800])
+@pytest.mark.parametrize("N1", [16, 32])
+def test_large_first_token_is_the_reference_of_every_wave(N1, S1, dtype):
+    """A first token 24 binades above the rest (an attention sink), and one
+    token 20 binades above the rest in each later quarter of the positions:
+    relative to the first token no numerator passes 1, relative to a later
+    quarter's own first tokens the fp16 one of its large token is infinite.
+    One token dominates, so the output is bounded by one rounding of P."""
+    import dsa_triton_ascend_amd as dsa
+    print(f"[few heads] sink N1={N1} S1={S1} {dtype}", flush=True)
+    K = 1024
+    level = np.zeros(K, np.float32)
+    level[0] = 24
+    level[[300, 600, 1000]] = 20
+    q, k, qr, kr = sfa_inputs(1, S1, K, N1, D, dtype, scale_qk=0.25, seed=11)
+    qr[..., 0] = 8.0
+    scale = 1.0 / np.sqrt(D + 64)
+    kr[0, :, 0, 0] = torch.from_numpy(level / (8.0 * scale * 1.4426950408889634)).to(dtype).float().numpy()
+    si = np.broadcast_to(np.arange(K, dtype=np.int32), (1, S1, 1, K)).copy()
+    got = dsa.sparse_flash_attention_triton(
+        dev(q, dtype), dev(k, dtype), None, dev(si, torch.int32), scale_value=scale, query_rope=dev(qr, dtype),
+        key_rope=dev(kr, dtype), sparse_mode=0, return_softmax_lse=True)
+    torch.cuda.synchronize()
+    rows = [0, S1 // 2, S1 - 1]
+    ref = sfa_fwd_bsnd(q, k, si, qr, kr, scale, [S1], [K], 1, 0, True, "float32", positions="kernel",
+                       rows=[(0, r) for r in rows])
+    for g, e, name in zip(got, ref, ("out", "softmax_max", "softmax_sum")):
+        ax = 1 if name == "out" else 2
+        atol = 2.0 ** -9 * float(np.abs(k).max()) if name == "out" else 2e-3
+        assert_close(np.take(g.float().cpu().numpy(), rows, ax), np.take(e, rows, ax), 2e-2, atol, name)
