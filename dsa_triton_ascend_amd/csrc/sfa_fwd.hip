@@ -28,6 +28,7 @@
 //  * When there are fewer rows than CUs the row's tokens are split across
 //    workgroups (all on one XCD) and a combine kernel merges the partial
 //    (O, max, sum) triples.
+#include <algorithm>
 #include <atomic>
 #include <mutex>
 #include <type_traits>
@@ -1507,10 +1508,18 @@ constexpr int kSfaFewMaxHeads = 32;  // up to here D = 512 runs sfa_fwd_few.hip
 // CUs, enough splits to fill them, with at least 256 positions per split.
 // From half the CUs up one split per unit: two splits of half the work
 // would take the same two rounds on the CUs, plus the merge.  A split's
-// range has no length limit (it is compacted in chunks), so the split
-// workspace is below (cus + units) <= 1.5 * cus partial rows of N1 heads
-// (about 51 MB at 256 CUs, N1 = 128, D = 512).  The workspace query and the
-// launch use the same count.
+// range has no length limit (it is compacted in chunks), so these splits are
+// at most CUs units of partials at D = 512 and 256 and 1.5 * CUs at D = 128
+// (17 MB at 256 CUs); D = 512 may take more to keep a range in one list
+// (sfa_fwd_splits_for).  The workspace query and the launch use the same
+// count.
+//
+// One round: where a CU holds one workgroup (D = 512, 256) the splits are at
+// most CUs / units, as one workgroup more starts a second round: 48 rows of
+// 16 heads, D = 512, 2048 tokens in five splits each 29.3 us; in six, 288
+// workgroups took 45.8 us; D = 256, 100 rows in two splits 54.0 us, in three
+// 75.2.  At D = 128 several workgroups share a CU, and the splits round up:
+// 100 rows of 16 heads in three splits each 32.4 us, in two 41.9.
 //
 // Kernel choice: D = 512 launches that split tokens with 64-head workgroups
 // run sfa_fwd_ds_kernel with 64 heads (decode: 44.8 us against 46.6 with
@@ -1519,16 +1528,18 @@ constexpr int kSfaFewMaxHeads = 32;  // up to here D = 512 runs sfa_fwd_few.hip
 // heads run sfa_fwd_few_kernel; other D = 512 launches run 128 heads per
 // workgroup (each KV row gathered once per row; prefill 4.64 ms against 4.77
 // for sfa_fwd_kernel); D < 512 runs sfa_fwd_kernel (128 heads).
-static int sfa_fwd_plan_splits(int64_t rows, int64_t n1, int64_t total_pos, int heads_per_wg) {
-  const int cus = device_cu_count();
-  const int64_t units = rows * ((n1 + heads_per_wg - 1) / heads_per_wg);
+static int64_t sfa_fwd_round_splits(int64_t units, int64_t total_pos, bool up) {
+  const int64_t cus = device_cu_count();
   if (2 * units > cus) return 1;
-  // one round of workgroups: 48 rows of 64 heads in 5 splits each 35 us; in 6,
-  // 288 workgroups took two rounds and 55 us
-  const int64_t want = cus / units;
+  const int64_t want = up ? (cus + units - 1) / units : cus / units;
   const int64_t by_len = (total_pos + 255) / 256;
-  const int64_t splits = want < by_len ? want : by_len;
-  return splits < 1 ? 1 : (int)splits;
+  return std::max<int64_t>(1, std::min(want, by_len));
+}
+static int64_t sfa_fwd_units(int64_t rows, int64_t n1, int heads_per_wg) {
+  return rows * ((n1 + heads_per_wg - 1) / heads_per_wg);
+}
+static int sfa_fwd_plan_splits(int64_t rows, int64_t n1, int64_t d, int64_t total_pos, int heads_per_wg) {
+  return (int)sfa_fwd_round_splits(sfa_fwd_units(rows, n1, heads_per_wg), total_pos, d < 256);
 }
 
 // ---------------------------------------------------------------------------
@@ -1536,9 +1547,9 @@ static int sfa_fwd_plan_splits(int64_t rows, int64_t n1, int64_t total_pos, int 
 // fixed-size device array instead of a caller's workspace, for callers that
 // cannot allocate (code under HIP graph capture, serving loops that forbid
 // hipMalloc).  Every GPU the library runs on holds its own copy until the
-// process ends.  64 MiB covers the split workspace of every shape on a
-// 256-CU device (at most 1.5 * CUs partial rows of N1 <= 128 heads: about
-// 51 MB at D = 512); larger needs are rejected.  Calls on one GPU share the
+// process ends.  64 MiB covers the splits that fill a 256-CU device at every
+// shape (17 MB); a D = 512 launch whose one-list splits would pass it takes
+// those alone and runs long ranges in chunks; larger needs are rejected.  Calls on one GPU share the
 // array: concurrent calls on one device race.  Every partial a launch reads
 // is written by the same launch, so nothing needs clearing between calls.
 // ---------------------------------------------------------------------------
@@ -1580,7 +1591,7 @@ int sfa_fwd_scratch(void** ptr) {
 enum SfaFwdKind { kFwdWide, kFwdDs64, kFwdDs128, kFwdFew };
 static SfaFwdKind sfa_fwd_kind(int64_t rows, int64_t n1, int64_t d, int64_t total_pos) {
   if (d != 512 || (test_flags() & kTestFwdWide)) return kFwdWide;
-  if (sfa_fwd_plan_splits(rows, n1, total_pos, kSfaDsHeads) > 1) return kFwdDs64;
+  if (sfa_fwd_plan_splits(rows, n1, d, total_pos, kSfaDsHeads) > 1) return kFwdDs64;
   // few heads: enough rows, or enough tokens per row, for waves that work alone
   if (n1 <= kSfaFewMaxHeads && (total_pos > 512 || rows > 2ll * device_cu_count())) return kFwdFew;
   if (n1 <= kSfaDsHeads) return kFwdDs64;
@@ -1607,7 +1618,7 @@ static size_t sfa_fwd_ws_for(int64_t splits, int64_t rows, int64_t n1, int64_t d
 // launch whose extra partials would pass kSfaOneListMaxWs.
 constexpr size_t kSfaOneListMaxWs = 4ull << 30;
 static int sfa_fwd_splits_for(int64_t rows, int64_t n1, int64_t d, int64_t total_pos, bool one_list) {
-  const int fill = sfa_fwd_plan_splits(rows, n1, total_pos, sfa_fwd_heads_per_wg(rows, n1, d, total_pos));
+  const int fill = sfa_fwd_plan_splits(rows, n1, d, total_pos, sfa_fwd_heads_per_wg(rows, n1, d, total_pos));
   if (!one_list || d != 512 || (test_flags() & kTestFwdWide)) return fill;
   if (sfa_fwd_kind(rows, n1, d, total_pos) == kFwdFew) return fill;  // takes ranges of any length
   const int64_t need = (total_pos + kSfaMaxList - 1) / kSfaMaxList;
