@@ -85,16 +85,25 @@ __device__ __forceinline__ int sfa_load_id(const P& p, const int32_t* idx_row, i
   return idx_row[pos / p.bs];
 }
 
+// Whether position `pos` with index entry `id` is attended, and its token.
+template <typename P>
+__device__ __forceinline__ bool sfa_visible(const P& p, const RowInfo& ri, int id, int pos, int64_t* tok) {
+  if (id < 0) return false;
+  *tok = (int64_t)id * p.bs + (pos % p.bs);
+  if (*tok >= ri.hi || *tok < ri.lo) return false;
+  if (p.layout_kv == DSA_LAYOUT_PA_BSND) return *tok < (int64_t)p.max_blocks * p.page_size;
+  if (p.layout_kv == DSA_LAYOUT_BSND && *tok >= p.s2) return false;
+  return ri.kv_base + *tok < p.kv_rows;
+}
+
 // `tab` is the row's block-table row (PA_BSND), in global memory or staged
 // in LDS by the caller.
 template <typename P>
 __device__ __forceinline__ bool sfa_resolve_id(const P& p, const RowInfo& ri, int id, int pos, int* phys,
                                                const int32_t* tab) {
-  if (id < 0) return false;
-  int64_t tok = (int64_t)id * p.bs + (pos % p.bs);
-  if (tok >= ri.hi || tok < ri.lo) return false;
+  int64_t tok;
+  if (!sfa_visible(p, ri, id, pos, &tok)) return false;
   if (p.layout_kv == DSA_LAYOUT_PA_BSND) {
-    if (tok >= (int64_t)p.max_blocks * p.page_size) return false;
     // tok < ri.hi fits in 32 bits (a 64-bit division takes several times as long)
     const unsigned pg = (unsigned)tok / (unsigned)p.page_size;
     int blk = tab[pg];
@@ -102,10 +111,7 @@ __device__ __forceinline__ bool sfa_resolve_id(const P& p, const RowInfo& ri, in
     *phys = (blk < 0 || r >= p.kv_rows) ? -1 : (int)r;
     return true;
   }
-  if (p.layout_kv == DSA_LAYOUT_BSND && tok >= p.s2) return false;
-  int64_t r = ri.kv_base + tok;
-  if (r >= p.kv_rows) return false;
-  *phys = (int)r;
+  *phys = (int)(ri.kv_base + tok);
   return true;
 }
 

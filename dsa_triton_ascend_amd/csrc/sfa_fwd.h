@@ -34,6 +34,7 @@ struct SfaFwdParams {
   int64_t band_pre, band_next;  // pre_tokens / next_tokens clamped to +-kBandOpen
   int32_t max_blocks, page_size;
   int32_t splits, pos_per_split;
+  int32_t lo_range;   // > 0: the lo part's rule holds for ranges of this length (SfaLoProbe)
   int32_t row_shift;  // 2^row_shift consecutive rows go to one XCD in turn (sfa_block_row)
   float scale_log2;
   int32_t return_lse;  // 0: no statistics, 1: the statistics, 2: zeros
@@ -61,6 +62,44 @@ __device__ __forceinline__ int64_t sfa_block_row(const SfaFwdParams& p, int xcd,
 // of the softmax, far below the fp32-golden tolerance (atol 2e-3) at these
 // lengths, while for a handful of tokens it is not.
 constexpr int kLoSplitMinTokens = 256;
+
+// The same rule where a launch takes fewer, longer ranges than the split count
+// rounded up: P keeps its lo part wherever it would have it in that count's
+// ranges (of lo_range positions).  A workgroup drops it only if every position
+// of its own range is attended, and so are enough beyond both ends to fill the
+// first and the last of those ranges that it touches up to the limit: one
+// probed position per thread, loaded beside the workgroup's own (0.5 us per
+// launch; counting every touched range took 2, and the lo part in all
+// workgroups 4 of 29).
+template <int NTHR>
+struct SfaLoProbe {
+  static constexpr int kN = 2 * kLoSplitMinTokens / NTHR;
+  int pos[kN], id[kN];  // pos < 0: nothing to probe
+  template <typename P>
+  __device__ __forceinline__ void load(const P& p, const int32_t* idx_row, int p0, int p1, int tid) {
+    const int total = p.K * p.bs, r = p.lo_range;
+    const int end = (p1 - 1) / r * r + kLoSplitMinTokens;         // the last range's limit
+    const int beg = min(p1, p0 / r * r + r) - kLoSplitMinTokens;  // the first range's, from its end
+#pragma unroll
+    for (int u = 0; u < kN; ++u) {
+      const int i = u * NTHR + tid;
+      const int x = i < kLoSplitMinTokens ? p1 + i : p0 + kLoSplitMinTokens - 1 - i;
+      pos[u] = (i < kLoSplitMinTokens ? x < end : x >= max(beg, 0)) ? x : -1;
+      id[u] = pos[u] >= 0 && x < total ? sfa_load_id(p, idx_row, x) : -1;
+    }
+  }
+  // whether a position that this wave probed is not attended
+  template <typename P>
+  __device__ __forceinline__ bool missing(const P& p, const RowInfo& ri) const {
+    bool miss = false;
+#pragma unroll
+    for (int u = 0; u < kN; ++u) {
+      int64_t tok;
+      miss |= pos[u] >= 0 && !(ri.active && sfa_visible(p, ri, id[u], pos[u], &tok));
+    }
+    return __any(miss);
+  }
+};
 constexpr float kRefSlack = 64.f;  // log2 units
 // Smallest exponent of a split partial's scale 2^e: a partial whose largest
 // |O / l| is below 2^kPartMinExp (tiny values) keeps the scale 2^-120, so

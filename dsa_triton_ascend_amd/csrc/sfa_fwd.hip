@@ -93,6 +93,7 @@ __global__ __launch_bounds__(NW * 64, 1) void sfa_fwd_kernel(SfaFwdParams p) {
   // from LDS by GEMM1's last k-steps instead of held in registers
   __shared__ __attribute__((aligned(16))) unsigned char s_q[HEADS_PER_WG * QL * 64];
   __shared__ int s_wcnt[NW];
+  __shared__ int s_lo[NW];
   __shared__ RowInfo s_ri;  // the row's lengths, for compacting chunks after the first
 
   const int tid = threadIdx.x;
@@ -170,6 +171,10 @@ __global__ __launch_bounds__(NW * 64, 1) void sfa_fwd_kernel(SfaFwdParams p) {
   // ahead of anything they would issue now.
   const int n_chunks = p1 > p0 ? (CH ? (p1 - p0 + kSfaMaxList - 1) / kSfaMaxList : 1) : 0;
   const int first_id = p0 + tid < p1 ? sfa_load_id(p, idx_row, p0 + tid) : -1;
+  constexpr bool kLoRanges = kSplitP && D >= 256;  // D = 128 rounds its split count up
+  const bool lo_probed = kLoRanges && !CH && p.lo_range >= kLoSplitMinTokens;
+  SfaLoProbe<NTHR> probe;
+  if (lo_probed) probe.load(p, idx_row, p0, p1, tid);
   const int32_t* tab = nullptr;
   if (p.layout_kv == DSA_LAYOUT_PA_BSND) {
     const int32_t* gtab = p.block_table + (int64_t)ri.b * p.max_blocks;
@@ -235,7 +240,17 @@ __global__ __launch_bounds__(NW * 64, 1) void sfa_fwd_kernel(SfaFwdParams p) {
     const int cb = q0 + c * kSfaMaxList;
     compact_range(cb, min(q1, cb + kSfaMaxList), rc, p.idx + row2 * p.K, tb, false);
   };
+  if (lo_probed) {
+    const bool miss = probe.missing(p, ri);
+    if (lane == 0) s_lo[wave] = miss;  // ordered by compact's barriers
+  }
   if (n_chunks > 0) compact(0);
+  bool lo_short = kLoRanges && p.lo_range > 0;
+  if (lo_probed) {
+    lo_short = n_valid < p1 - p0;
+#pragma unroll
+    for (int w = 0; w < NW; ++w) lo_short |= s_lo[w] != 0;
+  }
 
   // ---- tile gather: global -> LDS by DMA, swizzled rows ----
   // nope: DMA i of wave w covers tokens (i*NW + w)*TPI .. +TPI, lane L holds
@@ -598,7 +613,7 @@ __global__ __launch_bounds__(NW * 64, 1) void sfa_fwd_kernel(SfaFwdParams p) {
   // are compacted here and issue their own first tiles
   for (int c = 0; c < (CH && n_chunks > 0 ? n_chunks : 1); ++c) {
     if (CH && c > 0) compact(c);
-    if (kSplitP && n_valid >= kLoSplitMinTokens) run_tiles(c > 0, LoOff{});
+    if (kSplitP && n_valid >= kLoSplitMinTokens && !lo_short) run_tiles(c > 0, LoOff{});
     else run_tiles(c > 0, LoOn{});
   }
   if (__syncthreads_or(overflow ? 1 : 0)) {
@@ -783,6 +798,8 @@ __global__ __launch_bounds__(512, 1) void sfa_fwd_ds_kernel(SfaFwdParams p) {
   float* const s_am = s_mref + HG;                           // [NW][HG]
   float* const s_mul = s_am + NW * HG;                       // [HG]
   __shared__ int s_wcnt[NW];
+  constexpr bool kLoRanges = kSplitP && HG == kSfaDsHeads;  // the launches that split rows
+  __shared__ int s_lo[NW];
   __shared__ RowInfo s_ri;
 
   const int tid = threadIdx.x;
@@ -845,6 +862,9 @@ __global__ __launch_bounds__(512, 1) void sfa_fwd_ds_kernel(SfaFwdParams p) {
       first_ids[u] = pos < ce0 ? sfa_load_id(p, idx_row, pos) : -1;
     }
   }
+  const bool lo_probed = kLoRanges && !CH && p.lo_range >= kLoSplitMinTokens;
+  SfaLoProbe<NTHR> probe;
+  if (lo_probed) probe.load(p, idx_row, p0, p1, tid);
   const int32_t* tab = nullptr;
   const bool paged = p.layout_kv == DSA_LAYOUT_PA_BSND;
   const int32_t* gtab = paged ? p.block_table + (int64_t)ri.b * p.max_blocks : nullptr;
@@ -923,7 +943,17 @@ __global__ __launch_bounds__(512, 1) void sfa_fwd_ds_kernel(SfaFwdParams p) {
     const int cb = q0 + c * kSfaMaxList;
     compact_range(cb, min(q1, cb + kSfaMaxList), rc, p.idx + row2 * p.K, tb, false);
   };
+  if (lo_probed) {
+    const bool miss = probe.missing(p, ri);
+    if (lane == 0) s_lo[wave] = miss;  // ordered by compact's barriers
+  }
   if (n_chunks > 0) compact(0);
+  bool lo_short = kLoRanges && p.lo_range > 0;
+  if (lo_probed) {
+    lo_short = n_valid < p1 - p0;
+#pragma unroll
+    for (int w = 0; w < NW; ++w) lo_short |= s_lo[w] != 0;
+  }
 
   // ---- tile gather by LDS-DMA, spread over all eight waves ----
   // Nope DMA j < NIW of wave w loads the 1 KB row of token j*8 + w; waves
@@ -1239,7 +1269,7 @@ __global__ __launch_bounds__(512, 1) void sfa_fwd_ds_kernel(SfaFwdParams p) {
     for (int ht = 0; ht < HGT; ++ht) acc_o[j][ht] = (f32x4){0.f, 0.f, 0.f, 0.f};
   for (int c = 0; c < (CH && n_chunks > 0 ? n_chunks : 1); ++c) {
     if (CH && c > 0) compact(c);
-    if (kSplitP && n_valid >= kLoSplitMinTokens) run_tiles(c > 0, LoOff{});
+    if (kSplitP && n_valid >= kLoSplitMinTokens && !lo_short) run_tiles(c > 0, LoOff{});
     else run_tiles(c > 0, LoOn{});
   }
   // exact maxima of the two halves (64 heads); the vote barrier orders them
@@ -1542,6 +1572,15 @@ static int sfa_fwd_plan_splits(int64_t rows, int64_t n1, int64_t d, int64_t tota
   return (int)sfa_fwd_round_splits(sfa_fwd_units(rows, n1, heads_per_wg), total_pos, d < 256);
 }
 
+// The length that the lo-part rule counts tokens over (SfaLoProbe): a launch
+// in fewer splits than the rounded-up count takes the ranges of that count, as
+// its own longer ones pass the limit where those would not (70 rows of 64
+// heads, 1000 tokens: three splits of 334 tokens for four of 250).
+static int32_t sfa_fwd_lo_range(int64_t rows, int64_t n1, int64_t total_pos, int heads_per_wg, int64_t splits) {
+  const int64_t up = sfa_fwd_round_splits(sfa_fwd_units(rows, n1, heads_per_wg), total_pos, true);
+  return splits < up ? (int32_t)((total_pos + up - 1) / up) : 0;
+}
+
 // ---------------------------------------------------------------------------
 // Scratch of dsa_sfa_fwd_noalloc: the split partials live in this
 // fixed-size device array instead of a caller's workspace, for callers that
@@ -1734,6 +1773,7 @@ int sfa_fwd_run(const void* query, const void* query_rope, const void* key, cons
   const SfaFwdKind kind = sfa_fwd_kind(q_rows, n1, d, total_pos);
   p.splits = sfa_fwd_splits_for(q_rows, n1, d, total_pos, one_list);
   p.pos_per_split = (int32_t)((total_pos + p.splits - 1) / p.splits);
+  p.lo_range = sfa_fwd_lo_range(q_rows, n1, total_pos, sfa_fwd_heads_per_wg(q_rows, n1, d, total_pos), p.splits);
   p.part_o = nullptr;
   p.part_ml = nullptr;
   if (p.splits > 1) {

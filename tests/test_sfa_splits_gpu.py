@@ -1,5 +1,7 @@
-"""The forward's token splits in bf16: at D = 128 their count rounds up, which keeps
-a range of 250 tokens below the limit of the numerators' lo part.
+"""The forward's token splits in bf16.  Launches with one workgroup per CU round
+the split count down; the softmax numerators keep their lo part wherever the
+rounded-up count's ranges hold fewer than 256 tokens, as they did in those
+ranges.
 
 With hi + lo numerators (16 bits) the output is the exact value but for the
 split partials' rounding to fp16, at most 2^-11 of their magnitude, before its
@@ -17,7 +19,13 @@ pytestmark = pytest.mark.gpu
 
 
 @pytest.mark.parametrize("rows,N1,D,K,up", [
+    (70, 64, 512, 1000, 0),    # three splits of 334 for four of 250
+    (48, 16, 512, 2048, 6),    # five of 410 for six of 342, 200 tokens in each of the six
+    (20, 128, 512, 2048, 7),   # six of 342 for seven of 293
+    (100, 16, 256, 2048, 3),   # two of 1024 for three of 683
+    (70, 128, 256, 1000, 0),
     (70, 16, 128, 1000, 0),    # four of 250: D = 128 rounds up
+    (100, 16, 512, 6000, 3),   # two of 3000 for three of 2000, in chunks of 2048 positions
 ])
 def test_numerators_keep_their_lo_part(rows, N1, D, K, up):
     import dsa_triton_ascend_amd as dsa
