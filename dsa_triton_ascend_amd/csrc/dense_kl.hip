@@ -48,6 +48,7 @@
 // max |dI| and max |w|) so that its hi / lo parts stay in the fp16 normal
 // range; products are scaled back in fp32.
 #include <algorithm>
+#include <type_traits>
 
 #include "kl_common.h"
 
@@ -245,7 +246,8 @@ constexpr int kDkTileBytes = kDkTile64 * kDkRowDi * 2;
 
 // Row r of a tile (256 bytes) holds its 16-byte chunk c at c ^ nope_swz(r).
 // Wave w of four issues rows 16 w .. 16 w + 15, four rows (1 KB) per DMA; rows
-// past the last one re-read it (their products are never used).
+// past the last one re-read it.  A tile may hold rows past the visible ones,
+// with anything in them: the kernels keep those out of their results.
 __device__ __forceinline__ void dk_issue_tile(unsigned lds, const unsigned char* base, int row0, int last, int wave,
                                               int lane) {
 #pragma unroll
@@ -908,12 +910,15 @@ __global__ __launch_bounds__(256) void dense_dki_reduce_kernel(const float* part
 // 32-row tile between two barriers the two kernels took 547 and 769 us at 4096
 // causal rows of 64 heads (here 382 and 536; 412 GFLOP each, hi and lo parts
 // counted).  c goes to the second product as
-// hi + lo parts.  One half tile (32 rows) at a time: 48 MFMAs.
+// hi + lo parts.  One half tile (32 rows) at a time: 48 MFMAs.  LIM: rows from
+// `lim` on count as zeros in both products (their dots and their c = 0 would
+// carry a NaN or an infinity that they hold into acc).
 constexpr int kDkCols = 32;
 
-template <typename T, bool SCALED, typename F>
+template <typename T, bool SCALED, bool LIM, typename F>
 __device__ __forceinline__ void dk_half_tile(const unsigned char* half, const typename Elem<T>::v8 (&res)[2][4],
-                                             f32x4 (&acc)[kDkRowDi / 16][2], float unscale, int li, int lg, F&& value) {
+                                             f32x4 (&acc)[kDkRowDi / 16][2], float unscale, int lim, int li, int lg,
+                                             F&& value) {
   using E = Elem<T>;
   using V8 = typename E::v8;
   constexpr int IROW = kDkRowDi * 2;
@@ -934,7 +939,8 @@ __device__ __forceinline__ void dk_half_tile(const unsigned char* half, const ty
   for (int c = 0; c < 2; ++c)
 #pragma unroll
     for (int j = 0; j < 8; ++j) {
-      const float v = value(c, j >> 2, j & 3, dot[c][j >> 2][j & 3]);
+      const bool in = !LIM || (j >> 2) * 16 + lg * 4 + (j & 3) < lim;
+      const float v = value(c, j >> 2, j & 3, in ? dot[c][j >> 2][j & 3] : 0.f);
       const T h = E::from_f32(v);
       hi[c][j] = h;
       lo[c][j] = E::from_f32(v - E::to_f32(h));
@@ -945,7 +951,11 @@ __device__ __forceinline__ void dk_half_tile(const unsigned char* half, const ty
     const unsigned char* p1 = half + r1 * IROW + (((2 * dt + hb) ^ nope_swz(r1)) * 16) + (li & 1) * 8;
     const i16x4 w1 = __builtin_bit_cast(i16x4, __builtin_amdgcn_ds_read_tr16_b64_v4bf16((lds_bf16x4*)p1));
     const i16x4 w2 = __builtin_bit_cast(i16x4, __builtin_amdgcn_ds_read_tr16_b64_v4bf16((lds_bf16x4*)(p1 + 16 * IROW)));
-    const i16x8 w = {w1[0], w1[1], w1[2], w1[3], w2[0], w2[1], w2[2], w2[3]};
+    i16x8 w = {w1[0], w1[1], w1[2], w1[3], w2[0], w2[1], w2[2], w2[3]};
+    if constexpr (LIM) {
+#pragma unroll
+      for (int j = 0; j < 8; ++j) w[j] = (j >> 2) * 16 + lg * 4 + (j & 3) < lim ? w[j] : (short)0;
+    }
     const V8 av = __builtin_bit_cast(V8, w);
 #pragma unroll
     for (int c = 0; c < 2; ++c) {
@@ -1017,6 +1027,16 @@ __global__ __launch_bounds__(256, 2) void dense_dqi_tile_kernel(DkParams p) {
   for (int dt = 0; dt < kDkRowDi / 16; ++dt)
 #pragma unroll
     for (int c = 0; c < 2; ++c) acc[dt][c] = (f32x4){0.f, 0.f, 0.f, 0.f};
+  auto half_tile = [&](const unsigned char* half, int hh, int lim, auto limited) {
+    f32x4 di[2];
+#pragma unroll
+    for (int tt = 0; tt < 2; ++tt) di[tt] = *(const f32x4*)&s_di[wave][hh * 32 + tt * 16 + lg * 4];
+    dk_half_tile<T, false, decltype(limited)::value>(half, res, acc, 1.f, lim, li, lg, [&](int c, int tt, int r, float dot) {
+      const float relu = relu_bits(dot);
+      dw[c] = fmaf(di[tt][r], relu, dw[c]);
+      return relu > 0.f ? di[tt][r] * wg[c] * scale : 0.f;
+    });
+  };
   int b3 = 0;
   for (int t = 0; t < nt; ++t) {
     s_di[wave][lane] = t * kDkTile64 + lane < vis ? di_raw : 0.f;
@@ -1025,20 +1045,21 @@ __global__ __launch_bounds__(256, 2) void dense_dqi_tile_kernel(DkParams p) {
     di_raw = irow[min((t + 1) * kDkTile64 + lane, p.s2 - 1)];
     const int bn = b3 == 0 ? 2 : b3 - 1;
     if (t + 2 < nt) dk_issue_tile(ring + bn * kDkTileBytes, kib, (t + 2) * kDkTile64, p.s2 - 1, wave, lane);
-    if (t * kDkTile64 < vis) {
+    if ((t + 1) * kDkTile64 <= vis) {
 #pragma unroll
-      for (int hh = 0; hh < 2; ++hh) {
-        f32x4 di[2];
-#pragma unroll
-        for (int tt = 0; tt < 2; ++tt) di[tt] = *(const f32x4*)&s_di[wave][hh * 32 + tt * 16 + lg * 4];
-        dk_half_tile<T, false>(s_t[b3] + hh * 32 * IROW, res, acc, 1.f, li, lg, [&](int c, int tt, int r, float dot) {
-          const float relu = relu_bits(dot);
-          dw[c] = fmaf(di[tt][r], relu, dw[c]);
-          return relu > 0.f ? di[tt][r] * wg[c] * scale : 0.f;
-        });
-      }
+      for (int hh = 0; hh < 2; ++hh) half_tile(s_t[b3] + hh * 32 * IROW, hh, 32, std::false_type{});
     }
     b3 = b3 == 2 ? 0 : b3 + 1;
+  }
+  // the wave's partial tile, the loop's last or the one before (the rows of a
+  // workgroup differ by fewer than 64 keys): both are still in the ring.  Here
+  // and not in the loop, which the limited code beside the other makes spill.
+  if (vis % kDkTile64) {
+    const int t = vis / kDkTile64;
+    s_di[wave][lane] = t * kDkTile64 + lane < vis ? irow[min(t * kDkTile64 + lane, p.s2 - 1)] : 0.f;
+#pragma unroll 1
+    for (int hh = 0; t * kDkTile64 + hh * 32 < vis; ++hh)
+      half_tile(s_t[t % 3] + hh * 32 * IROW, hh, vis - t * kDkTile64 - hh * 32, std::true_type{});
   }
   if (!have) return;
   typedef T T4 __attribute__((ext_vector_type(4)));
@@ -1162,7 +1183,7 @@ __global__ __launch_bounds__(256, 2) void dense_dki_tile_kernel(DkParams p) {
       f32x4 w[2];
 #pragma unroll
       for (int tt = 0; tt < 2; ++tt) w[tt] = *(const f32x4*)&s_w[t & 1][hh * 32 + tt * 16 + lg * 4];
-      dk_half_tile<T, kF16>(s_t[b3] + hh * 32 * IROW, res, acc, unscale, li, lg, [&](int c, int tt, int r, float dot) {
+      dk_half_tile<T, kF16, false>(s_t[b3] + hh * 32 * IROW, res, acc, unscale, 32, li, lg, [&](int c, int tt, int r, float dot) {
         return dot > 0.f ? dv[c] * w[tt][r] * scale : 0.f;
       });
     }

@@ -57,3 +57,39 @@ def test_weights_at_an_odd_offset(w_dtype):
     b = dsa.dense_loss_backward_triton(d[0], d[1], d[2], d[3], _dev(w, w_dtype), *st, **kw)
     for x, y in zip(a, b):
         assert np.array_equal(_np(x), _np(y))
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16], ids=["bf16", "fp16"])
+@pytest.mark.parametrize("Ni,Di", [(32, 128), (64, 128), (128, 128), (64, 256)])
+@pytest.mark.parametrize("bad", [float("nan"), float("inf"), -float("inf")])
+def test_key_rows_that_no_row_sees_are_not_read(bad, Ni, Di, dtype):
+    """Non-finite index keys past the key lengths (padding that nobody wrote)
+    change nothing: every output is bit for bit that of finite padding."""
+    print(f"[dense tiles] padding {bad} Ni={Ni} Di={Di} {dtype}", flush=True)
+    B, S1, S2 = 3, 70, 200
+    aq, ak = [70, 33, 5], [150, 20, 131]
+    c = list(_case(B, S1, S2, 32, 1, 128, Ni, Di, dtype, torch.float32, aq, ak))
+    want = _run(c, dtype, torch.float32, given_lse=False, act_q=aq, act_k=ak)
+    c[5] = c[5].copy()
+    for b in range(B):
+        c[5][b, ak[b]:] = bad
+    got = _run(c, dtype, torch.float32, given_lse=False, act_q=aq, act_k=ak)
+    for x, y in zip(got, want):
+        assert np.array_equal(x, y)
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16], ids=["bf16", "fp16"])
+@pytest.mark.parametrize("Ni", [32, 64, 128])
+@pytest.mark.parametrize("at", [64, 97, 129])
+def test_key_rows_behind_the_causal_diagonal(at, Ni, dtype):
+    """A NaN index key reaches the query rows that see it and no others (the
+    rows before it share its tile)."""
+    print(f"[dense tiles] diagonal at={at} Ni={Ni} {dtype}", flush=True)
+    S = 150
+    c = list(_case(1, S, S, 32, 1, 128, Ni, 128, dtype, torch.float32))
+    want = _run(c, dtype, torch.float32, given_lse=False)
+    c[5] = c[5].copy()
+    c[5][0, at] = float("nan")
+    got = _run(c, dtype, torch.float32, given_lse=False)
+    for i in (0, 2):  # dQueryIndex, dWeights
+        assert np.array_equal(got[i][0, :at], want[i][0, :at])
