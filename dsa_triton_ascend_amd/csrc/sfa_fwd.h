@@ -100,7 +100,11 @@ struct SfaLoProbe {
     return __any(miss);
   }
 };
-constexpr float kRefSlack = 64.f;  // log2 units
+// How far (log2 units) a score may pass a head's reference max: the numerators
+// 2^(s - m_ref) go to the second product in T, whose largest power of two is
+// 2^127 (bf16; the fp32 sums keep the rest of the range) or 2^15 (fp16).
+template <typename T> constexpr float kRefSlack = 64.f;
+template <> inline constexpr float kRefSlack<f16> = 15.f;
 // Smallest exponent of a split partial's scale 2^e: a partial whose largest
 // |O / l| is below 2^kPartMinExp (tiny values) keeps the scale 2^-120, so
 // the stored multiplier inv * 2^-e (inv <= 1: l counts the reference-max

@@ -403,8 +403,8 @@ __global__ __launch_bounds__(NW * 64, 1) void sfa_fwd_kernel(SfaFwdParams p) {
   // It is fixed by the first tile with a visible token and never raised
   // inside the tile loop (raising it would rescale O, which the register
   // allocator can only do by cycling the accumulator through VGPRs every
-  // tile).  P = 2^(s - m_ref) may therefore exceed 1; up to 2^kRefSlack is
-  // exact in fp32/bf16.  A head whose max exceeds m_ref + kRefSlack sets
+  // tile).  P = 2^(s - m_ref) may therefore exceed 1; up to 2^kRefSlack
+  // it is in range in T and in the fp32 sums.  A head whose max exceeds m_ref + kRefSlack sets
   // `overflow`, and the row is recomputed once with m_ref = exact max.
   // m_true tracks the exact max for the returned statistics.
 #pragma unroll
@@ -550,7 +550,7 @@ __global__ __launch_bounds__(NW * 64, 1) void sfa_fwd_kernel(SfaFwdParams p) {
       tmax = xgroup_max(tmax);
       m_true[ht] = fmaxf(m_true[ht], tmax);
       if (m_ref[ht] == -INFINITY) m_ref[ht] = tmax;
-      overflow |= tmax > m_ref[ht] + kRefSlack;
+      overflow |= tmax > m_ref[ht] + kRefSlack<T>;
       V8 hi, lo;
       float lsum = 0.f;
 #pragma unroll
@@ -1156,7 +1156,7 @@ __global__ __launch_bounds__(512, 1) void sfa_fwd_ds_kernel(SfaFwdParams p) {
       // first tile's with a visible score
       if (m_ref == -INFINITY) m_ref = tmax;
     }
-    overflow |= tmax > m_ref + kRefSlack;
+    overflow |= tmax > m_ref + kRefSlack<T>;
     float lsum = 0.f;
 #pragma unroll
     for (int u = 0; u < NTT; ++u) {

@@ -282,7 +282,7 @@ __global__ __launch_bounds__(TW * 64, 1) void sfa_fwd_few_kernel(SfaFwdParams p)
       const float tmax = scaled(s, ht, nleft, v);
       m_true[ht] = fmaxf(m_true[ht], tmax);
       if (!exact_ref && m_ref[ht] == -INFINITY) m_ref[ht] = tmax;
-      overflow |= tmax > m_ref[ht] + kRefSlack;
+      overflow |= tmax > m_ref[ht] + kRefSlack<T>;
 #pragma unroll
       for (int r = 0; r < 4; ++r) {
         const float e = m_ref[ht] == -INFINITY ? 0.f : fast_exp2(v[r] - m_ref[ht]);
