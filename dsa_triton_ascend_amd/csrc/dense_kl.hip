@@ -266,14 +266,31 @@ __device__ __forceinline__ void dk_wait_tile(bool next_in_flight) {
   else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
 }
 
+// xgroup_sum in 64 bits
+__device__ __forceinline__ double xgroup_sum64(double v) {
+  typedef unsigned u32x2 __attribute__((ext_vector_type(2)));
+  u32x2 b = __builtin_bit_cast(u32x2, v);
+  auto l = __builtin_amdgcn_permlane16_swap(b[0], b[0], false, false);
+  auto h = __builtin_amdgcn_permlane16_swap(b[1], b[1], false, false);
+  v = __builtin_bit_cast(double, (u32x2){l[0], h[0]}) + __builtin_bit_cast(double, (u32x2){l[1], h[1]});
+  b = __builtin_bit_cast(u32x2, v);
+  l = __builtin_amdgcn_permlane32_swap(b[0], b[0], false, false);
+  h = __builtin_amdgcn_permlane32_swap(b[1], b[1], false, false);
+  return __builtin_bit_cast(double, (u32x2){l[0], h[0]}) + __builtin_bit_cast(double, (u32x2){l[1], h[1]});
+}
+
 // Index scores I and their LSE at D_idx = 128: one query row per wave, four
 // consecutive rows of a batch per workgroup sharing each 64-key tile.  A row's
 // NHT * 16 heads are resident MFMA A operands, so a key fragment read from LDS
 // feeds NHT products (one, in dense_index_kernel, whose eight waves split the
 // heads of one row: its LDS reads and three barriers per 32 keys took 459 us
-// at 4096 causal rows of 64 heads, this takes 125 us, 137 GFLOP: 1.1 PFLOP/s).  The
+// at 4096 causal rows of 64 heads, this takes 131 us, 137 GFLOP: 1.05 PFLOP/s).  The
 // weighted ReLU head sum runs on the accumulators in fp32, the four 16-lane
 // groups' partial sums meet in two lane swaps, and lane l ends up with key l.
+// Those last two additions are in 64 bits: at the scores' full size, their
+// fp32 rounding was a third of the scores' error (over 300 to 4096 rows of 32
+// to 128 heads the LSE's sum was off by 1.8e-6 to 3.6e-6, now 1.6e-6 to 2.9e-6;
+// the three-part product of dense_index_kernel 2.0e-6 to 4.4e-6).  3 of 131 us.
 template <int NHT, typename T>
 __global__ __launch_bounds__(256, NHT > 4 ? 2 : 3) void dense_index_rows_kernel(DkParams p) {
   using E = Elem<T>;
@@ -347,7 +364,7 @@ __global__ __launch_bounds__(256, NHT > 4 ? 2 : 3) void dense_index_rows_kernel(
         for (int ht = 0; ht < NHT; ++ht)
 #pragma unroll
           for (int r = 0; r < 4; ++r) a[r] = fmaf(relu_bits(acc[ht][r]), wr[ht][r], a[r]);
-        const float sum = xgroup_sum((a[0] + a[1]) + (a[2] + a[3]));
+        const float sum = (float)xgroup_sum64((a[0] + a[1]) + (a[2] + a[3]));
         I = lg == kt ? sum : I;
       }
       const int key = t * kDkTile64 + lane;

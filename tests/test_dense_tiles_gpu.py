@@ -3,6 +3,8 @@ tiles, 128-key workgroups and query-row chunks: lengths around the tile sizes,
 several rows per workgroup, more keys than queries and the reverse, batches
 with hidden rows, 16-bit weights at an odd element offset.  Oracle, tolerances
 and their reasons: test_dense_kl_gpu."""
+import math
+
 import numpy as np
 import pytest
 import torch
@@ -93,3 +95,29 @@ def test_key_rows_behind_the_causal_diagonal(at, Ni, dtype):
     got = _run(c, dtype, torch.float32, given_lse=False)
     for i in (0, 2):  # dQueryIndex, dWeights
         assert np.array_equal(got[i][0, :at], want[i][0, :at])
+
+
+def test_index_lse_is_as_exact_as_its_scores():
+    """The LSE's sum is off by the scores' absolute error.  Scores of 32 heads
+    with weights in [0, 1) are about 72; rounded once to fp32 from sums of a
+    quarter each they are off by 3.1e-8 of that (2.4e-8 from the last rounding,
+    the rest from the quarters), 2.25e-6."""
+    import dsa_triton_ascend_amd as dsa
+    print("[dense tiles] LSE error", flush=True)
+    S, Ni, dt = 3001, 32, torch.float16
+    g = torch.Generator(device="cuda").manual_seed(7)
+    qi = torch.randn(1, S, Ni, 128, generator=g, device="cuda", dtype=dt)
+    ki = torch.randn(1, S, 1, 128, generator=g, device="cuda", dtype=dt)
+    w = torch.rand(1, S, Ni, generator=g, device="cuda")
+    mx, sm = dsa.dense_lightning_indexer_softmax_lse_triton(qi, ki, w)
+    kt = ki[0, :, 0].double().t().contiguous()
+    exp = torch.empty(S, dtype=torch.float64, device="cuda")
+    for a in range(0, S, 128):
+        b = min(S, a + 128)
+        relu = (qi[0, a:b].double().reshape(-1, 128) @ kt).reshape(b - a, Ni, S).clamp_(min=0)
+        score = (relu * w[0, a:b].double()[..., None]).sum(1)
+        score.masked_fill_(torch.arange(S, device="cuda")[None] > torch.arange(a, b, device="cuda")[:, None], -math.inf)
+        exp[a:b] = (score - score.max(1, keepdim=True).values).exp().sum(1)
+    err = ((sm.double().reshape(-1) - exp).norm() / exp.norm()).item()
+    print(f"[dense tiles] sum off by {err:.3g}", flush=True)
+    assert err < 2.25e-6
