@@ -197,9 +197,10 @@ def dense_loss_backward_triton(query, key, query_index, key_index, weights, soft
         sm = _row_stat(softmax_sum_index, B, S1, "softmax_sum_index")
     act_q = _seq_tensor(actual_seq_qlen, device)
     act_k = _seq_tensor(actual_seq_klen, device)
-    d_qi = torch.empty_like(query_index)
-    d_ki = torch.empty_like(key_index)
-    d_w = torch.empty_like(weights)
+    # the kernels write rows in order, whatever the input's strides
+    d_qi = torch.empty_like(query_index, memory_format=torch.contiguous_format)
+    d_ki = torch.empty_like(key_index, memory_format=torch.contiguous_format)
+    d_w = torch.empty_like(weights, memory_format=torch.contiguous_format)
     loss = torch.empty(1, dtype=torch.float32, device=device)
     lib = _lib.load()
     ws_bytes = lib.dsa_dense_kl_bwd_workspace_size(B, S1, S2, D_idx)

@@ -123,10 +123,11 @@ def _sfa_grad(query, key, value, sparse_indices, d_out, out, softmax_max, softma
         raise ValueError("actual sequence length arrays must have one entry per batch")
     _check_device(query, key, query_rope, key_rope, sparse_indices, d_out, out, softmax_max, softmax_sum)
 
-    dq = torch.empty_like(query)
-    dqr = torch.empty_like(query_rope)
-    dk = torch.empty_like(key)
-    dkr = torch.empty_like(key_rope)
+    # the kernels write rows in order, whatever the input's strides
+    dq = torch.empty_like(query, memory_format=torch.contiguous_format)
+    dqr = torch.empty_like(query_rope, memory_format=torch.contiguous_format)
+    dk = torch.empty_like(key, memory_format=torch.contiguous_format)
+    dkr = torch.empty_like(key_rope, memory_format=torch.contiguous_format)
     if value is not None and value.dtype != key.dtype:
         raise ValueError("value dtype must equal the key dtype")
     dv = None if merge_kv else torch.empty(key.shape, dtype=key.dtype, device=device)

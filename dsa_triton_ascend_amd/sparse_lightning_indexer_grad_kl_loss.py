@@ -145,9 +145,10 @@ def sparse_lightning_indexer_grad_kl_loss_triton(
             or softmax_sum.numel() != q_rows * N1 or weights.numel() != q_rows * Nidx1:
         raise ValueError("sparse_indices / softmax statistics / weights do not match the query rows")
 
-    d_qi = torch.empty_like(query_index)
-    d_ki = torch.empty_like(key_index)
-    d_w = torch.empty_like(weights)
+    # the kernels write rows in order, whatever the input's strides
+    d_qi = torch.empty_like(query_index, memory_format=torch.contiguous_format)
+    d_ki = torch.empty_like(key_index, memory_format=torch.contiguous_format)
+    d_w = torch.empty_like(weights, memory_format=torch.contiguous_format)
     loss = torch.empty(1, dtype=torch.float32, device=device)
     lib = _lib.load()
     if layout_k == "BSND" and not tnd:
