@@ -21,7 +21,7 @@
 //  * dense_index_rows_kernel (D_idx = 128): four query rows per workgroup, one
 //    per wave, over shared 64-key tiles.  Writes I to a row-major fp32 buffer
 //    [rows, S2] and the row's LSE (online per lane, merged at the end).
-//  * dense_index_kernel (D_idx = 256, 512): one workgroup per query row streams
+//  * dense_index_kernel (D_idx = 256, 512, unaligned rows): one workgroup per query row streams
 //    the visible key index rows through LDS; 16 index heads per wave on MFMA,
 //    the weighted ReLU head-sum as an exact three-part bf16 product with a ones
 //    matrix.
@@ -1267,8 +1267,16 @@ int dense_kl_splits(int64_t batch, int64_t s1, int64_t s2) {
   return (int)sp;
 }
 
-// The tile kernels take D_idx = 128 and whole 32-head groups that divide four.
-static bool dk_tiles(int64_t nidx, int64_t di) { return di == kDkRowDi && (nidx == 32 || nidx == 64 || nidx == 128); }
+// The D_idx = 128 kernels stage rows by 16-byte LDS-DMA, whose source must be
+// aligned; rows at another address (a view that starts at an odd element) run
+// the kernels that load them through registers.  dQi, dW and dKi take whole
+// 32-head groups that divide four.
+static bool dk_rows(const DkParams& p, int64_t di) {
+  return di == kDkRowDi && (((uintptr_t)p.qi | (uintptr_t)p.ki) & 15) == 0;
+}
+static bool dk_tiles(const DkParams& p, int64_t di) {
+  return dk_rows(p, di) && (p.nidx == 32 || p.nidx == 64 || p.nidx == 128);
+}
 
 // Query rows per dKi workgroup, at least 32: one round of two workgroups per
 // CU over the (key tile, visible rows) of full-length sequences, counting a
@@ -1322,12 +1330,13 @@ size_t dense_kl_workspace_bytes(int64_t batch, int64_t s1, int64_t s2, int64_t d
 template <typename T>
 static hipError_t dk_index(const DkParams& p, int di, hipStream_t stream) {
   const dim3 grid((unsigned)(p.batch * p.s1));
-  if (di == kDkRowDi) {
+  if (dk_rows(p, di)) {
     const dim3 g4((unsigned)(p.batch * (((int64_t)p.s1 + 3) / 4)));
     if (p.nidx <= 32) hipLaunchKernelGGL((dense_index_rows_kernel<2, T>), g4, dim3(256), 0, stream, p);
     else if (p.nidx <= 64) hipLaunchKernelGGL((dense_index_rows_kernel<4, T>), g4, dim3(256), 0, stream, p);
     else hipLaunchKernelGGL((dense_index_rows_kernel<8, T>), g4, dim3(256), 0, stream, p);
-  } else if (di == 256) hipLaunchKernelGGL((dense_index_kernel<256, T>), grid, dim3(kDkThreads), 0, stream, p);
+  } else if (di == 128) hipLaunchKernelGGL((dense_index_kernel<128, T>), grid, dim3(kDkThreads), 0, stream, p);
+  else if (di == 256) hipLaunchKernelGGL((dense_index_kernel<256, T>), grid, dim3(kDkThreads), 0, stream, p);
   else hipLaunchKernelGGL((dense_index_kernel<512, T>), grid, dim3(kDkThreads), 0, stream, p);
   return hipGetLastError();
 }
@@ -1352,7 +1361,7 @@ static hipError_t dk_grads(const DkParams& p, int di, void* d_key_index, hipStre
   const dim3 rgrid((unsigned)(p.batch * p.s1)), blk(kDkThreads);
   const int64_t ntiles = (p.s2 + kDkKeys - 1) / kDkKeys;
   const dim3 kgrid((unsigned)(p.batch * ntiles * p.splits));
-  if (dk_tiles(p.nidx, di)) {
+  if (dk_tiles(p, di)) {
     const int rpw = 4 / (p.nidx / kDkCols);
     hipLaunchKernelGGL((dense_dqi_tile_kernel<T>), dim3((unsigned)(p.batch * (((int64_t)p.s1 + rpw - 1) / rpw))), dim3(256), 0,
                        stream, p);

@@ -121,3 +121,23 @@ def test_index_lse_is_as_exact_as_its_scores():
     err = ((sm.double().reshape(-1) - exp).norm() / exp.norm()).item()
     print(f"[dense tiles] sum off by {err:.3g}", flush=True)
     assert err < 2.25e-6
+
+
+@pytest.mark.parametrize("which", ["query_index", "key_index"])
+def test_index_rows_at_an_odd_offset(which):
+    """Index rows that start two bytes past a 16-byte boundary."""
+    import dsa_triton_ascend_amd as dsa
+    print(f"[dense tiles] odd offset {which}", flush=True)
+    dt = torch.bfloat16
+    c = _case(1, 66, 140, 32, 1, 128, 64, 128, dt, torch.float32)
+    q, k, qr, kr, qi, ki, w, smax, ssum, scale = c
+    t = {"query_index": _dev(qi, dt), "key_index": _dev(ki, dt)}
+    buf = torch.empty(t[which].numel() + 1, dtype=dt, device="cuda")
+    odd = buf[1:].view(t[which].shape)
+    odd.copy_(t[which])
+    t[which] = odd
+    assert odd.is_contiguous() and odd.data_ptr() % 16 == 2
+    got = dsa.dense_loss_backward_triton(
+        _dev(q, dt), _dev(k, dt), t["query_index"], t["key_index"], _dev(w, torch.float32), _dev(smax, torch.float32),
+        _dev(ssum, torch.float32), scale_value=scale, query_rope=_dev(qr, dt), key_rope=_dev(kr, dt))
+    _check([_np(x) for x in got], dense_kl_bwd(q, k, qr, kr, qi, ki, w, smax, ssum, scale), which, torch.float32)
