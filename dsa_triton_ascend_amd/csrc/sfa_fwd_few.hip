@@ -83,7 +83,7 @@ __global__ __launch_bounds__(TW * 64, 1) void sfa_fwd_few_kernel(SfaFwdParams p)
   __shared__ __attribute__((aligned(1024))) unsigned char smem[TW][2 * BUFB];
   __shared__ int s_list[TW][LIST];
   __shared__ float s_st[TW > 1 ? TW : 1][3][HEADS];
-  __shared__ float s_ref[HEADS];
+  __shared__ float s_ref[TW][HEADS];
   __shared__ int s_cnt[TW], s_tiles[TW];
 
   const int tid = threadIdx.x;
@@ -393,57 +393,61 @@ __global__ __launch_bounds__(TW * 64, 1) void sfa_fwd_few_kernel(SfaFwdParams p)
     }
   };
 
-  // ---- the reference maxima, from the row's first two tiles: the first wave
-  // with a tile in its first chunk scores them for all.  (Before the
-  // accumulators are in use: beside them a second copy of the product made
-  // the 32-head kernels spill.)
+  // ---- the reference maxima: the row's first two tiles, scored once for them
+  // alone, before the accumulators are in use.  Every wave scores its own, and
+  // all take those of the first wave that has any.
   int n_others = 0;  // tokens of the other waves' first chunks
   const bool last0 = p0 + kFewChunk >= p1;
-  bool primed = false;  // tile 1 is on its way whole
   if (p0 < p1) open_chunk(p0, last0);
-  bool first = nt > 0;
+  bool primed = nt > 1;  // tile 1 is on its way whole
+  if (primed) {
+#pragma unroll
+    for (int j = 0; j < 4; ++j) issue_nope(r1, 1, 3, j);
+  }
+#pragma unroll 1
+  for (int t = 0; t < min(nt, 2); ++t) {
+    if (t == 0 && primed) wait_vmcnt<NDMA>();  // tile 1's
+    else wait_vmcnt<0>();
+    f32x4 s[HT][2];
+    gemm1(t, s, false, r1);
+#pragma unroll
+    for (int ht = 0; ht < HT; ++ht) {
+      float v[4];
+      m_ref[ht] = fmaxf(m_ref[ht], scaled(s, ht, n_list - t * TILE, v));
+    }
+  }
   if constexpr (TW > 1) {
     if (lane == 0) {
       s_cnt[wave] = n_total;
       s_tiles[wave] = nt;
     }
-    lds_barrier();
+    if (lg == 0) {
 #pragma unroll
-    for (int w = 0; w < TW; ++w) {
+      for (int ht = 0; ht < HT; ++ht) s_ref[wave][ht * 16 + li] = m_ref[ht];
+    }
+    lds_barrier();
+    int from = 0;
+#pragma unroll
+    for (int w = TW - 1; w >= 0; --w) {
       n_others += w == wave ? 0 : s_cnt[w];
-      first = first && (w >= wave || s_tiles[w] == 0);
+      from = s_tiles[w] > 0 ? w : from;
     }
+#pragma unroll
+    for (int ht = 0; ht < HT; ++ht) m_ref[ht] = s_ref[from][ht * 16 + li];
   }
-  if (first) {
-    primed = nt > 1;
-    if (primed) {
+
+  // Q in VGPRs from here on: left to one register class with the use above,
+  // these kernels spilled it (up to 950 bytes of scratch per lane: 17 us more
+  // per launch of 130 rows; the others do not, and are 3 % slower with this)
+  if constexpr (HT == 2 && (TW > 1 || !BUF)) {
 #pragma unroll
-      for (int j = 0; j < 4; ++j) issue_nope(r1, 1, 3, j);
-    }
-#pragma unroll 1
-    for (int t = 0; t < min(nt, 2); ++t) {
-      if (t == 0 && primed) wait_vmcnt<NDMA>();  // tile 1's
-      else wait_vmcnt<0>();
-      f32x4 s[HT][2];
-      gemm1(t, s, false, r1);
+    for (int ht = 0; ht < HT; ++ht)
 #pragma unroll
-      for (int ht = 0; ht < HT; ++ht) {
-        float v[4];
-        m_ref[ht] = fmaxf(m_ref[ht], scaled(s, ht, n_list - t * TILE, v));
+      for (int ks = 0; ks < KS; ++ks) {
+        u32x4 x = as_u4(qf[ht][ks]);
+        asm volatile("" : "+v"(x));
+        qf[ht][ks] = as_v8<V8>(x);
       }
-    }
-  }
-  if constexpr (TW > 1) {
-    if (first && lg == 0) {
-#pragma unroll
-      for (int ht = 0; ht < HT; ++ht) s_ref[ht * 16 + li] = m_ref[ht];
-    }
-    lds_barrier();
-    bool any = false;
-#pragma unroll
-    for (int w = 0; w < TW; ++w) any = any || s_tiles[w] > 0;
-#pragma unroll
-    for (int ht = 0; ht < HT; ++ht) m_ref[ht] = any ? s_ref[ht * 16 + li] : -INFINITY;
   }
 
   // A head whose scores pass the reference max by more than the slack sends
