@@ -9,7 +9,7 @@ import numpy as np
 import pytest
 import torch
 
-from oracle.dense_kl import dense_kl_bwd
+from oracle.dense_kl import dense_index_lse, dense_kl_bwd
 from tests.test_dense_kl_gpu import _case, _check, _dev, _np, _run
 
 pytestmark = pytest.mark.gpu
@@ -141,3 +141,38 @@ def test_index_rows_at_an_odd_offset(which):
         _dev(q, dt), _dev(k, dt), t["query_index"], t["key_index"], _dev(w, torch.float32), _dev(smax, torch.float32),
         _dev(ssum, torch.float32), scale_value=scale, query_rope=_dev(qr, dt), key_rope=_dev(kr, dt))
     _check([_np(x) for x in got], dense_kl_bwd(q, k, qr, kr, qi, ki, w, smax, ssum, scale), which, torch.float32)
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16], ids=["bf16", "fp16"])
+@pytest.mark.parametrize("Ni", [1, 48, 100])
+def test_head_counts_of_the_c_interface(Ni, dtype):
+    """Index head counts that the library takes and the Python API does not:
+    partly filled head tiles of the scores, and the per-row gradient kernels."""
+    from dsa_triton_ascend_amd import _lib
+    print(f"[dense tiles] C interface Ni={Ni} {dtype}", flush=True)
+    B, S1, S2, N1, D = 2, 40, 150, 32, 128
+    aq, ak = [40, 17], [150, 77]
+    c = _case(B, S1, S2, N1, 1, D, Ni, 128, dtype, torch.float32, aq, ak)
+    q, k, qr, kr, qi, ki, w, smax, ssum, scale = c
+    d = [_dev(x, dtype) for x in (q, k, qr, kr, qi, ki)] + [_dev(x, torch.float32) for x in (w, smax, ssum)]
+    seq = [torch.tensor(x, dtype=torch.int32, device="cuda") for x in (aq, ak)]
+    outs = [torch.empty_like(d[4]), torch.empty_like(d[5]), torch.empty_like(d[6]), torch.empty(1, device="cuda")]
+    imax, isum = torch.empty(B, S1, device="cuda"), torch.empty(B, S1, device="cuda")
+    lib, stream = _lib.load(), _lib.stream_handle(torch.device("cuda", torch.cuda.current_device()))
+    n = lib.dsa_dense_kl_bwd_workspace_size(B, S1, S2, 128)
+    ws = torch.empty(n, dtype=torch.uint8, device="cuda")
+    code, f32 = _lib.dtype_code(dtype), _lib.dtype_code(torch.float32)
+    p = [t.data_ptr() for t in d]
+    _lib.check(lib.dsa_dense_li_softmax_lse(p[4], p[5], p[6], seq[0].data_ptr(), seq[1].data_ptr(), imax.data_ptr(),
+                                            isum.data_ptr(), B, S1, S2, Ni, 128, code, f32, stream), "lse")
+    _lib.check(lib.dsa_dense_kl_bwd(
+        p[0], p[1], p[2], p[3], p[4], p[5], p[6], p[7], p[8], imax.data_ptr(), isum.data_ptr(), seq[0].data_ptr(),
+        seq[1].data_ptr(), *[t.data_ptr() for t in outs], B, S1, S2, N1, 1, D, 64, Ni, 128, code, f32, scale,
+        ws.data_ptr(), n, stream), "bwd")
+    torch.cuda.synchronize()
+    em, es = dense_index_lse(qi, ki, w, act_q=aq, act_k=ak)
+    rows = es.reshape(B, S1) > 0
+    np.testing.assert_allclose(_np(imax)[rows], em.reshape(B, S1)[rows], rtol=1e-5, atol=1e-4)
+    np.testing.assert_allclose(_np(isum), es.reshape(B, S1), rtol=1e-4, atol=1e-2)
+    exp = dense_kl_bwd(q, k, qr, kr, qi, ki, w, smax, ssum, scale, act_q=aq, act_k=ak)
+    _check([_np(x) for x in outs], exp, f"Ni={Ni}", torch.float32)
