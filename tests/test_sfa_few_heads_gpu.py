@@ -182,3 +182,10 @@ def test_large_first_token_is_the_reference_of_every_wave(N1, S1, dtype):
         ax = 1 if name == "out" else 2
         atol = 2.0 ** -9 * float(np.abs(k).max()) if name == "out" else 2e-3
         assert_close(np.take(g.float().cpu().numpy(), rows, ax), np.take(e, rows, ax), 2e-2, atol, name)
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16], ids=["bf16", "fp16"])
+@pytest.mark.parametrize("S1,N1,K", [(140, 64, 1000), (600, 64, 300), (130, 32, 640), (260, 32, 768)])
+def test_whole_rows_on_the_64_head_kernel(S1, N1, K, dtype):
+    """Unsplit rows of 64 heads, and of 32 heads with few tokens each."""
+    _check(S1, S1 + 1500, N1, K, 3, dtype)
