@@ -1633,10 +1633,10 @@ static SfaFwdKind sfa_fwd_kind(int64_t rows, int64_t n1, int64_t d, int64_t tota
   if (sfa_fwd_plan_splits(rows, n1, d, total_pos, kSfaDsHeads) > 1) return kFwdDs64;
   // Few heads: enough rows, or enough tokens per row, for waves that work
   // alone.  Up to two rows per CU four waves share a row, and their start and
-  // merge weigh more than the padding of short rows (bf16, us, few heads
-  // against 64; 130 rows of 16 heads: 256 positions 18.5 / 18.2, 512 23.6 /
-  // 28.1, and at 300 rows 37.8 / 34.5, 47.8 / 53.8; 32 heads: 512 34.7 / 29.2,
-  // 640 37.8 / 34.6, 768 41 / 39.8, 1024 47.1 / 49.5).  With more rows the line is gone (513 rows of
+  // merge weigh more than the padding of short rows (us, few heads against 64;
+  // 130 rows of 16 heads, bf16: 256 positions 18.5 / 18.2, 512 23.6 / 28.1, and
+  // at 300 rows 37.8 / 34.5, 47.8 / 53.8; 32 heads, fp16: 640 36.0 / 35.0, 800
+  // 40.2 / 41.3, 1024 44.3 / 49.9).  With more rows the line is gone (513 rows of
   // 32 heads, 64 positions: 23.0 / 31.6, 512: 61.9 / 81.0).
   if (n1 <= kSfaFewMaxHeads && (total_pos > (n1 <= 16 ? 512 : 768) || rows > 2ll * device_cu_count())) return kFwdFew;
   if (n1 <= kSfaDsHeads) return kFwdDs64;

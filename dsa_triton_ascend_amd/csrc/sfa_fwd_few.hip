@@ -9,10 +9,12 @@
 // workgroups of eight waves with two workgroup barriers per 32-token tile; at
 // 32 heads three quarters of their MFMAs multiplied zeros and a tile still
 // took 4.2 k cycles.  Measured (one MI355X, through the Python API): 8192
-// causal rows of 2048 tokens, 16 / 32 heads 3.88 / 3.92 -> 1.18 / 1.43 ms; a
-// packed batch of 5247 rows of up to 1024 tokens, 32 heads 1.34 -> 0.43 ms
-// (10.2 TB/s of gathered rows; the same loop without the softmax, on rows that
-// stay in L2, reaches 15.5).
+// causal rows of 2048 tokens, 16 / 32 heads 3.87 / 3.89 -> 1.24 / 1.43 ms; a
+// packed batch of 5247 rows of up to 1024 tokens, 32 heads 1.34 -> 0.44 ms
+// (10 TB/s of gathered rows; the same loop without the softmax, on rows that
+// stay in L2, reaches 15.5).  The 32-head kernels spill 2 to 19 registers (12 to
+// 80 bytes of scratch per lane; 36 to 74, 116 to 188 bytes, with the 64-bit
+// gather), none of them inside the tile loop.
 //
 // Here every wave works alone: it takes its own range of index positions,
 // compacts them, gathers 16-token tiles by LDS-DMA into its own two-buffer
@@ -91,12 +93,8 @@ __global__ __launch_bounds__(TW * 64, 1) void sfa_fwd_few_kernel(SfaFwdParams p)
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int li = lane & 15, lg = lane >> 4;
 
-  const int hgroups = (p.n1 + HEADS - 1) / HEADS;
-  const int jj = (int)(blockIdx.x >> 3);
-  const int hg = jj % hgroups;
-  const int64_t row = sfa_block_row(p, (int)(blockIdx.x & 7), jj / hgroups);
+  const int64_t row = sfa_block_row(p, (int)(blockIdx.x & 7), (int)(blockIdx.x >> 3));  // n1 <= HEADS
   if (row < 0) return;
-
 
   // ---- this wave's positions ----
   const RowInfo ri = sfa_row_info(p, (int)row);
@@ -117,12 +115,11 @@ __global__ __launch_bounds__(TW * 64, 1) void sfa_fwd_few_kernel(SfaFwdParams p)
   asm volatile("" ::: "memory");  // the index entries go out before Q
 
   // ---- Q (B operand of S^T): lane -> head li of each head tile, k = 8 lg .. ----
-  const int head0 = hg * HEADS;
   V8 qf[HT][KS];
   const u32x4 z4 = {0u, 0u, 0u, 0u};
 #pragma unroll
   for (int ht = 0; ht < HT; ++ht) {
-    const int head = head0 + ht * 16 + li;
+    const int head = ht * 16 + li;
     const bool hv = head < p.n1;
     const int64_t hs = row * p.n1 + (hv ? head : 0);
 #pragma unroll
@@ -229,7 +226,10 @@ __global__ __launch_bounds__(TW * 64, 1) void sfa_fwd_few_kernel(SfaFwdParams p)
     };
 #pragma unroll
     for (int ht = 0; ht < HT; ++ht) s[ht][0] = s[ht][1] = (f32x4){0.f, 0.f, 0.f, 0.f};
-    constexpr int PF = 6;  // K fragments in flight
+    // K fragments in flight; with six, the bf16 kernel for 32 heads and four
+    // waves copies an accumulator tile between register files in its loop (700
+    // rows of 2048 tokens 256 us against 211)
+    constexpr int PF = HT == 2 && TW > 1 && kSplitP && BUF ? 4 : 6;
     V8 fa[PF];
 #pragma unroll
     for (int i = 0; i < PF; ++i) fa[i] = kfrag(i);
@@ -503,7 +503,7 @@ __global__ __launch_bounds__(TW * 64, 1) void sfa_fwd_few_kernel(SfaFwdParams p)
 #pragma unroll
     for (int ht = 0; ht < HT; ++ht) {
       mul[ht] = l_run[ht] > 0.f ? 1.f / l_run[ht] : 0.f;
-      const int head = head0 + ht * 16 + li;
+      const int head = ht * 16 + li;
       if (p.return_lse && lg == 0 && head < p.n1) {
         const bool any = p.return_lse == 1 && l_run[ht] > 0.f;
         p.smax[row * p.n1 + head] = any ? m_true[ht] * kLn2 : 0.f;
@@ -528,7 +528,7 @@ __global__ __launch_bounds__(TW * 64, 1) void sfa_fwd_few_kernel(SfaFwdParams p)
 #pragma unroll
     for (int h = 0; h < HEADS; ++h) {
       const u32x4 v = *(const u32x4*)(ring + h * SROW + lane * 16);
-      if (head0 + h < p.n1) *(u32x4*)((unsigned char*)p.out + (row * p.n1 + head0 + h) * (D * 2) + lane * 16) = v;
+      if (h < p.n1) *(u32x4*)((unsigned char*)p.out + (row * p.n1 + h) * (D * 2) + lane * 16) = v;
     }
   } else {
     // merge the waves in fp32 through the idle rings: O_w counts 2^(m_ref_w - M)
@@ -589,8 +589,8 @@ __global__ __launch_bounds__(TW * 64, 1) void sfa_fwd_few_kernel(SfaFwdParams p)
     }
 #pragma unroll
     for (int i = 0; i < HPW; ++i) {
-      const int h = wave * HPW + i, head = head0 + h;
-      if (head >= p.n1) break;
+      const int h = wave * HPW + i;
+      if (h >= p.n1) break;
       const float M = top(h);
       float L = 0.f, mt = -INFINITY;
 #pragma unroll
@@ -599,7 +599,7 @@ __global__ __launch_bounds__(TW * 64, 1) void sfa_fwd_few_kernel(SfaFwdParams p)
         mt = fmaxf(mt, s_st[w][2][h]);
       }
       const float inv = L > 0.f ? 1.f / L : 0.f;
-      const int64_t orow = row * p.n1 + head;
+      const int64_t orow = row * p.n1 + h;
 #pragma unroll
       for (int u = 0; u < 2; ++u) {
         const f32x4 v = res[i][u] * inv;
@@ -627,15 +627,15 @@ int sfa_few_heads_per_wg(int64_t n1) { return n1 <= 16 ? 16 : 32; }
 
 hipError_t sfa_few_launch(const SfaFwdParams& p, int32_t dtype, bool buf, int64_t rows_per_xcd, hipStream_t stream) {
   const int hpw = sfa_few_heads_per_wg(p.n1);
-  const int64_t hgroups = (p.n1 + hpw - 1) / hpw;
-  const unsigned blocks = (unsigned)(8 * rows_per_xcd * hgroups);
+  const unsigned blocks = (unsigned)(8 * rows_per_xcd);
   // One wave per row once the rows come near filling every SIMD (16 heads,
-  // 2048 tokens: 166 against 195 us at 1000 rows); below that a workgroup's
-  // four waves share a row's tokens (700 rows: 146 against 165 us).  With
-  // short rows, whose start and merge weigh more, the line lies lower (700
-  // causal rows of up to 512 tokens: 47 against 61 us).
+  // 2048 tokens: 179 against 229 us at 800 rows); below that a workgroup's
+  // four waves share a row's tokens (600 rows: 173 against 176 us; 1024 tokens,
+  // 500 rows 74 against 92).  With short rows, whose start and merge weigh more,
+  // the line lies lower (700 causal rows of up to 512 tokens: one wave 50 us,
+  // four 65; 1024 tokens: 95 and 108).
   const int64_t per_cu = (int64_t)p.K * p.bs <= 1024 ? 2 : 3;
-  const bool one = p.rows * hgroups > per_cu * device_cu_count();
+  const bool one = p.rows > per_cu * device_cu_count();
   auto go = [&](auto t) {
     using T = decltype(t);
     if (hpw == 16) one ? launch_one<T, 1, 1>(p, buf, blocks, stream) : launch_one<T, 1, 4>(p, buf, blocks, stream);
