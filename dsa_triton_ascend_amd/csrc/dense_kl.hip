@@ -925,7 +925,7 @@ __global__ __launch_bounds__(256) void dense_dki_reduce_kernel(const float* part
 // fragment read from LDS, plain or transposed, feeds two column tiles, and a
 // workgroup's four waves share the tile; with 16 columns per wave and one
 // 32-row tile between two barriers the two kernels took 547 and 769 us at 4096
-// causal rows of 64 heads (here 382 and 536; 412 GFLOP each, hi and lo parts
+// causal rows of 64 heads (here 361 and 534; 412 GFLOP each, hi and lo parts
 // counted).  c goes to the second product as
 // hi + lo parts.  One half tile (32 rows) at a time: 48 MFMAs.  LIM: rows from
 // `lim` on count as zeros in both products (their dots and their c = 0 would

@@ -145,8 +145,8 @@ size_t dsa_sfa_fwd_workspace_size(int64_t q_rows, int64_t n1, int64_t d,
  * capturing this entry point into a HIP graph).  Rows longer than one index
  * list whose split partials would exceed 64 MiB run one split per row
  * through the chunked kernel instead; sizes whose workspace still exceeds
- * 64 MiB are rejected with DSA_ERR_UNSUPPORTED (on a 256-CU MI355X no
- * supported shape needs more than about 51 MB).  The array is shared by
+ * 64 MiB are rejected with DSA_ERR_UNSUPPORTED (on a 256-CU MI355X the
+ * splits that fill the device need at most 17 MB).  The array is shared by
  * every call on a GPU: calls that overlap on one device (concurrent streams
  * or threads) race and must be serialised by the caller.
  */
