@@ -1680,13 +1680,17 @@ size_t sfa_fwd_workspace_bytes(int64_t rows, int64_t n1, int64_t d, int64_t tota
   return sfa_fwd_ws_for(sfa_fwd_splits_for(rows, n1, d, total_pos, one_list), rows, n1, d);
 }
 
-// Rows that go to one XCD in turn: 32 (one per CU of an XCD, so the rounds of
-// the CUs stay even), and below 256 rows the largest power of two that gives
-// every XCD the same number of rows.
+// Rows that go to one XCD in turn: up to 32 (one per CU of an XCD, so the
+// rounds of the CUs stay even), the largest power of two that leaves no XCD
+// more than an eighth above the mean (300 rows of 128 heads, 32 tokens: 38 rows
+// per XCD 31.0 us; in blocks of 32, two XCDs with 64 and the others with 32,
+// 33.1; in blocks of 8 30.8), and below 256 rows the largest that gives every
+// XCD the same number of rows.
 static int sfa_row_shift(int64_t rows) {
   const int64_t rpx = (rows + 7) / 8;
+  auto slots = [&](int sh) { return ((rpx + (1ll << sh) - 1) >> sh) << sh; };  // of the fullest XCD
   int sh = 0;
-  while (sh < 5 && (rows >= 256 || rpx % (2ll << sh) == 0)) ++sh;
+  while (sh < 5 && (rows >= 256 ? 64 * slots(sh + 1) <= 9 * rows : slots(sh + 1) == rpx)) ++sh;
   return sh;
 }
 static int64_t sfa_rows_per_xcd(const SfaFwdParams& p) {

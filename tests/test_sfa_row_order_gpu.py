@@ -28,3 +28,10 @@ def test_every_row_is_computed_once(S1, D, N1):
     ref = sfa_fwd_bsnd(q, k, si, qr, kr, scale, [S1], [S1], 1, 3, True, "float32", positions="kernel")
     for g, e, name in zip(got, ref, ("out", "softmax_max", "softmax_sum")):
         assert_close(g.float().cpu().numpy(), e, 2e-2, 2e-3, name)
+
+
+@pytest.mark.parametrize("S1", [264, 400, 513, 600, 800])
+def test_every_row_is_computed_once_in_smaller_blocks(S1):
+    """Counts whose blocks of rows are smaller than 32, to keep the XCDs even."""
+    test_every_row_is_computed_once(S1, 512, 128)
+    test_every_row_is_computed_once(S1, 128, 4)
