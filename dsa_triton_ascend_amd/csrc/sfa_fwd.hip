@@ -1548,8 +1548,12 @@ constexpr int kSfaFewMaxHeads = 32;  // up to here D = 512 runs sfa_fwd_few.hip
 // most CUs / units, as one workgroup more starts a second round: 48 rows of
 // 16 heads, D = 512, 2048 tokens in five splits each 29.3 us; in six, 288
 // workgroups took 45.8 us; D = 256, 100 rows in two splits 54.0 us, in three
-// 75.2.  At D = 128 several workgroups share a CU, and the splits round up:
-// 100 rows of 16 heads in three splits each 32.4 us, in two 41.9.
+// 75.2.  Where the rows do not spread evenly enough over the XCDs for one
+// round, more and shorter splits are better again: 17 rows of 128 heads, three
+// on one XCD, in eight splits 47.6 us, in seven 51.3; 33 rows of 16 heads 38.0
+// and 42.8.  So they are at D = 128,
+// where several workgroups share a CU: 100 rows of 16 heads in three splits each
+// 32.4 us, in two 41.9.
 //
 // Kernel choice: D = 512 launches that split tokens with 64-head workgroups
 // run sfa_fwd_ds_kernel with 64 heads (decode: 44.8 us against 46.6 with
@@ -1569,7 +1573,11 @@ static int64_t sfa_fwd_units(int64_t rows, int64_t n1, int heads_per_wg) {
   return rows * ((n1 + heads_per_wg - 1) / heads_per_wg);
 }
 static int sfa_fwd_plan_splits(int64_t rows, int64_t n1, int64_t d, int64_t total_pos, int heads_per_wg) {
-  return (int)sfa_fwd_round_splits(sfa_fwd_units(rows, n1, heads_per_wg), total_pos, d < 256);
+  const int64_t units = sfa_fwd_units(rows, n1, heads_per_wg);
+  const int64_t down = sfa_fwd_round_splits(units, total_pos, false);
+  const int64_t per_xcd = (rows + 7) / 8 * (units / rows) * down;  // workgroups of the fullest XCD
+  const bool one_round = d >= 256 && 8 * per_xcd <= device_cu_count();
+  return (int)(one_round ? down : sfa_fwd_round_splits(units, total_pos, true));
 }
 
 // The length that the lo-part rule counts tokens over (SfaLoProbe): a launch

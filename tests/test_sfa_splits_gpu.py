@@ -21,7 +21,8 @@ pytestmark = pytest.mark.gpu
 @pytest.mark.parametrize("rows,N1,D,K,up", [
     (70, 64, 512, 1000, 0),    # three splits of 334 for four of 250
     (48, 16, 512, 2048, 6),    # five of 410 for six of 342, 200 tokens in each of the six
-    (20, 128, 512, 2048, 7),   # six of 342 for seven of 293
+    (20, 128, 512, 2048, 7),   # seven of 293: six would take an XCD two rounds as well
+    (48, 128, 512, 2048, 3),   # two of 1024 for three of 683
     (100, 16, 256, 2048, 3),   # two of 1024 for three of 683
     (70, 128, 256, 1000, 0),
     (70, 16, 128, 1000, 0),    # four of 250: D = 128 rounds up
