@@ -1562,8 +1562,7 @@ constexpr int kSfaFewMaxHeads = 32;  // up to here D = 512 runs sfa_fwd_few.hip
 // heads run sfa_fwd_few_kernel; other D = 512 launches run 128 heads per
 // workgroup (each KV row gathered once per row; prefill 4.64 ms against 4.77
 // for sfa_fwd_kernel); D < 512 runs sfa_fwd_kernel (128 heads).
-static int64_t sfa_fwd_round_splits(int64_t units, int64_t total_pos, bool up) {
-  const int64_t cus = device_cu_count();
+static int64_t sfa_fwd_round_splits(int64_t cus, int64_t units, int64_t total_pos, bool up) {
   if (2 * units > cus) return 1;
   const int64_t want = up ? (cus + units - 1) / units : cus / units;
   const int64_t by_len = (total_pos + 255) / 256;
@@ -1573,11 +1572,12 @@ static int64_t sfa_fwd_units(int64_t rows, int64_t n1, int heads_per_wg) {
   return rows * ((n1 + heads_per_wg - 1) / heads_per_wg);
 }
 static int sfa_fwd_plan_splits(int64_t rows, int64_t n1, int64_t d, int64_t total_pos, int heads_per_wg) {
-  const int64_t units = sfa_fwd_units(rows, n1, heads_per_wg);
-  const int64_t down = sfa_fwd_round_splits(units, total_pos, false);
+  const int64_t cus = device_cu_count(), units = sfa_fwd_units(rows, n1, heads_per_wg);
+  if (2 * units > cus) return 1;
+  const int64_t down = d >= 256 ? sfa_fwd_round_splits(cus, units, total_pos, false) : 0;
   const int64_t per_xcd = (rows + 7) / 8 * (units / rows) * down;  // workgroups of the fullest XCD
-  const bool one_round = d >= 256 && 8 * per_xcd <= device_cu_count();
-  return (int)(one_round ? down : sfa_fwd_round_splits(units, total_pos, true));
+  const bool one_round = down > 0 && 8 * per_xcd <= cus;
+  return (int)(one_round ? down : sfa_fwd_round_splits(cus, units, total_pos, true));
 }
 
 // The length that the lo-part rule counts tokens over (SfaLoProbe): a launch
@@ -1585,7 +1585,8 @@ static int sfa_fwd_plan_splits(int64_t rows, int64_t n1, int64_t d, int64_t tota
 // its own longer ones pass the limit where those would not (70 rows of 64
 // heads, 1000 tokens: three splits of 334 tokens for four of 250).
 static int32_t sfa_fwd_lo_range(int64_t rows, int64_t n1, int64_t total_pos, int heads_per_wg, int64_t splits) {
-  const int64_t up = sfa_fwd_round_splits(sfa_fwd_units(rows, n1, heads_per_wg), total_pos, true);
+  if (splits == 1) return 0;  // then the rounded-up count is one as well
+  const int64_t up = sfa_fwd_round_splits(device_cu_count(), sfa_fwd_units(rows, n1, heads_per_wg), total_pos, true);
   return splits < up ? (int32_t)((total_pos + up - 1) / up) : 0;
 }
 
@@ -1791,7 +1792,7 @@ int sfa_fwd_run(const void* query, const void* query_rope, const void* key, cons
   const SfaFwdKind kind = sfa_fwd_kind(q_rows, n1, d, total_pos);
   p.splits = sfa_fwd_splits_for(q_rows, n1, d, total_pos, one_list);
   p.pos_per_split = (int32_t)((total_pos + p.splits - 1) / p.splits);
-  p.lo_range = sfa_fwd_lo_range(q_rows, n1, total_pos, sfa_fwd_heads_per_wg(q_rows, n1, d, total_pos), p.splits);
+  p.lo_range = sfa_fwd_lo_range(q_rows, n1, total_pos, kind == kFwdDs64 ? kSfaDsHeads : kSfaHeadsPerWg, p.splits);
   p.part_o = nullptr;
   p.part_ml = nullptr;
   if (p.splits > 1) {
